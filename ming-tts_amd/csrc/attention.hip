@@ -15,6 +15,7 @@
 //     partial sums meet in LDS in a fixed order.
 // Batched decode (mt_attention_decode) is the same kernel with a per-row cache base and
 // the row's query position read from a device array.
+#include "attend_row.hpp"
 #include "mt_device.hpp"
 #include "mt_internal.hpp"
 #include "mingtts_hip.h"
@@ -22,19 +23,6 @@
 namespace mt {
 
 namespace {
-
-constexpr int ATT_THREADS = 256;
-constexpr int ATT_MAXKEYS = 4096;
-
-template <int CT>
-__device__ __forceinline__ float4 load4(const void *base, size_t off) {
-    if constexpr (CT == DT_F32) {
-        return *reinterpret_cast<const float4 *>(static_cast<const float *>(base) + off);
-    } else {
-        const uint2 v = *reinterpret_cast<const uint2 *>(static_cast<const uint16_t *>(base) + off);
-        return make_float4(dec_lo<CT>(v.x), dec_hi<CT>(v.x), dec_lo<CT>(v.y), dec_hi<CT>(v.y));
-    }
-}
 
 template <int CT>
 __device__ __forceinline__ void store1(void *base, size_t off, float v) {
@@ -97,56 +85,13 @@ __global__ __launch_bounds__(256) void rope_cache_kernel(float *qkv, uint32_t ld
     }
 }
 
-// Max / sum over the 64 lanes, the same bits in every lane: quad swaps and the half-row and
-// row mirrors on DPP (rows of 16), then two exchanges between rows.
-__device__ __forceinline__ float wave_max(float v) {
-    v = fmaxf(v, dpp_mov<0xB1>(v));
-    v = fmaxf(v, dpp_mov<0x4E>(v));
-    v = fmaxf(v, dpp_mov<0x141>(v));
-    v = fmaxf(v, dpp_mov<0x140>(v));
-    v = fmaxf(v, __shfl_xor(v, 16, 64));
-    return fmaxf(v, __shfl_xor(v, 32, 64));
-}
-__device__ __forceinline__ float wave_sum(float v) { return group_sum(v, 64); }
-
-// The 16-byte raw loads of eight cached values (one of fp16, two of fp32) and their decode.
-template <int CT>
-struct Raw8 {
-    uint4 a, b;
-};
-template <int CT>
-__device__ __forceinline__ Raw8<CT> load8_raw(const void *base, size_t off) {
-    Raw8<CT> r;
-    if constexpr (CT == DT_F32) {
-        const uint4 *p = reinterpret_cast<const uint4 *>(static_cast<const float *>(base) + off);
-        r.a = p[0];
-        r.b = p[1];
-    } else {
-        r.a = *reinterpret_cast<const uint4 *>(static_cast<const uint16_t *>(base) + off);
-        r.b = make_uint4(0u, 0u, 0u, 0u);
-    }
-    return r;
-}
-template <int CT>
-__device__ __forceinline__ void decode8(const Raw8<CT> &r, float *o) {
-    if constexpr (CT == DT_F32) {
-        o[0] = __uint_as_float(r.a.x); o[1] = __uint_as_float(r.a.y); o[2] = __uint_as_float(r.a.z); o[3] = __uint_as_float(r.a.w);
-        o[4] = __uint_as_float(r.b.x); o[5] = __uint_as_float(r.b.y); o[6] = __uint_as_float(r.b.z); o[7] = __uint_as_float(r.b.w);
-    } else {
-        unpack8<CT>(r.a, o);
-    }
-}
-
 template <int CT>
 __global__ __launch_bounds__(ATT_THREADS) void attention_kernel(const float *q, uint32_t ldq, uint32_t hq,
                                                                 uint32_t hkv, uint32_t pos0, const uint32_t *lens,
                                                                 uint32_t window, const void *kc, const void *vc,
                                                                 uint32_t cache_len, uint64_t cache_stride,
                                                                 float *out, uint32_t ldo, float scale) {
-    __shared__ float sc[ATT_MAXKEYS];
-    __shared__ float red[ATT_THREADS / 64];
-    __shared__ float4 part[16][16];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    __shared__ RowLds lds;
     const uint32_t m = blockIdx.x / hq, h = blockIdx.x % hq;
     const uint32_t kvh = h / (hq / hkv);
     // Device-side lengths are clamped to the cache; a zero length attends to nothing and
@@ -158,95 +103,8 @@ __global__ __launch_bounds__(ATT_THREADS) void attention_kernel(const float *q, 
     const int nk = static_cast<int>(jEnd - jStart);
     const size_t kvbase = cbase + (static_cast<size_t>(kvh) * cache_len + jStart) * 64;
 
-    // Scores.
-    const int r = tid & 7;
-    float qf[8];
-    {
-        const float4 *qp = reinterpret_cast<const float4 *>(q + static_cast<size_t>(m) * ldq + h * 64 + 8 * r);
-        const float4 a = qp[0], b = qp[1];
-        qf[0] = a.x; qf[1] = a.y; qf[2] = a.z; qf[3] = a.w;
-        qf[4] = b.x; qf[5] = b.y; qf[6] = b.z; qf[7] = b.w;
-    }
-    // Sixteen passes of 32 keys per round, all requested before any is used (keys past the
-    // end re-read the last key and are skipped).
-    float mx = -INFINITY;
-    constexpr int KP = ATT_THREADS / 8, KU = 16;
-    for (int t0 = tid >> 3; t0 < nk; t0 += KU * KP) {
-        Raw8<CT> kr[KU];
-#pragma unroll
-        for (int u = 0; u < KU; u++) {
-            const int t = min(t0 + u * KP, nk - 1);
-            kr[u] = load8_raw<CT>(kc, kvbase + static_cast<size_t>(t) * 64 + 8 * r);
-        }
-#pragma unroll
-        for (int u = 0; u < KU; u++) {
-            const int t = t0 + u * KP;
-            if (t < nk) {  // the 8 lanes of a key agree
-                float kf[8];
-                decode8<CT>(kr[u], kf);
-                float s = 0.0f;
-#pragma unroll
-                for (int e = 0; e < 8; e++) s = fmaf(qf[e], kf[e], s);
-                s = octet_sum(s);
-                s *= scale;
-                if (r == 0) sc[t] = s;
-                mx = fmaxf(mx, s);
-            }
-        }
-    }
-    mx = wave_max(mx);
-    if (lane == 0) red[wave] = mx;
-    __syncthreads();
-    mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-    __syncthreads();
-
-    // Softmax numerators and their sum.
-    float sum = 0.0f;
-    for (int t = tid; t < nk; t += ATT_THREADS) {
-        const float e = exp_hw(sc[t] - mx);
-        sc[t] = e;
-        sum += e;
-    }
-    sum = wave_sum(sum);
-    if (lane == 0) red[wave] = sum;
-    __syncthreads();
-    sum = (red[0] + red[1]) + (red[2] + red[3]);
-
-    // p . v: 16 lanes per V row (4 dims each), 16 key phases, keys t = ks, ks + 16, ... in
-    // order; 32 rows per round requested before any is used (rows past the end re-read
-    // the last row and are skipped).
-    const int d4 = tid & 15, ks = tid >> 4;
-    constexpr int VU = 32;
-    float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    for (int t0 = ks; t0 < nk; t0 += 16 * VU) {
-        float4 v[VU];
-#pragma unroll
-        for (int u = 0; u < VU; u++)
-            v[u] = load4<CT>(vc, kvbase + static_cast<size_t>(min(t0 + 16 * u, nk - 1)) * 64 + 4 * d4);
-#pragma unroll
-        for (int u = 0; u < VU; u++) {
-            const int t = t0 + 16 * u;
-            if (t < nk) {
-                const float p = sc[t];
-                acc.x = fmaf(p, v[u].x, acc.x);
-                acc.y = fmaf(p, v[u].y, acc.y);
-                acc.z = fmaf(p, v[u].z, acc.z);
-                acc.w = fmaf(p, v[u].w, acc.w);
-            }
-        }
-    }
-    part[ks][d4] = acc;
-    __syncthreads();
-    if (tid < 16) {
-        float4 o = part[0][tid];
-        for (int k = 1; k < 16; k++) {
-            const float4 pp = part[k][tid];
-            o.x += pp.x; o.y += pp.y; o.z += pp.z; o.w += pp.w;
-        }
-        const float inv = sum > 0.0f ? 1.0f / sum : 0.0f;
-        float4 res = make_float4(o.x * inv, o.y * inv, o.z * inv, o.w * inv);
-        *reinterpret_cast<float4 *>(out + static_cast<size_t>(m) * ldo + h * 64 + 4 * tid) = res;
-    }
+    attend_row<CT, 16, 32>(q + static_cast<size_t>(m) * ldq + h * 64, kc, vc, kvbase, nk, scale,
+                           out + static_cast<size_t>(m) * ldo + h * 64, lds.sc, lds.red, lds.part);
 }
 
 // attention_kernel's arithmetic for R consecutive rows of one sequence at a time, for rows whose
@@ -678,10 +536,25 @@ int launch_rope_cache(float *qkv, uint32_t ldq, uint32_t rows, uint32_t hq, uint
     return check_launch("rope_cache");
 }
 
+// Rows of one sequence that go by 32-row blocks on the matrix cores (attention_mfma.hip).  Up to
+// 64 rows (mt_rope_attention's range) and, without a window, up to 256 keys or 320 fp16 rows the
+// row kernels are kept: there their results are those of the rows attended one call each, bit for
+// bit, and with an fp32 cache they are as fast (174 rows 7.6 against 7.7 us).  Above, graph replay,
+// row kernels against the matrix cores, fp16 / fp32 cache: 512 rows 21.4 / 21.2 against 7.4 / 11.7
+// us, 2048 rows 431 / 766 against 31 / 64 us, window 65: 100 rows 12.2 / 17.4 against 4.7 / 5.5
+// us, 1600 rows 132 / 233 against 10.1 / 12.4 us.
+static bool attention_tiles(uint32_t rows, uint32_t pos0, uint32_t window, int ct) {
+    if (rows <= 64) return false;
+    if (window > 0 && pos0 + rows > window) return true;
+    return ct == DT_F32 ? pos0 + rows > 256 : rows >= 320;
+}
+
 int launch_attention(const float *q, uint32_t ldq, uint32_t rows, uint32_t hq, uint32_t hkv, uint32_t pos0,
                      const uint32_t *lens, uint32_t window, const void *kc, const void *vc, int ct,
                      uint32_t cache_len, uint64_t cache_stride, float *out, uint32_t ldo, float scale,
                      hipStream_t stream) {
+    if (!lens && attention_tiles(rows, pos0, window, ct))
+        return launch_attention_mfma(q, ldq, rows, hq, hkv, pos0, window, kc, vc, ct, cache_len, out, ldo, scale, stream);
     // Rows of one sequence whose keys all start at position 0 go by blocks of AR_ROWS rows.
     if (!lens && rows >= AR_MIN_ROWS && pos0 + rows <= static_cast<uint32_t>(AR_MAXKEYS) &&
         (window == 0 || pos0 + rows <= window)) {

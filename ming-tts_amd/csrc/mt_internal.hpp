@@ -132,6 +132,10 @@ int launch_attention(const float *q, uint32_t ldq, uint32_t rows, uint32_t hq, u
                      const uint32_t *lens, uint32_t window, const void *kc, const void *vc, int ct,
                      uint32_t cache_len, uint64_t cache_stride, float *out, uint32_t ldo, float scale,
                      hipStream_t stream);
+// The same for rows of one sequence on the matrix cores (attention_mfma.hip).
+int launch_attention_mfma(const float *q, uint32_t ldq, uint32_t rows, uint32_t hq, uint32_t hkv, uint32_t pos0,
+                          uint32_t window, const void *kc, const void *vc, int ct, uint32_t cache_len, float *out,
+                          uint32_t ldo, float scale, hipStream_t stream);
 
 int launch_dit_attention(const float *qkv, uint32_t ld, uint32_t B, uint32_t S, uint32_t H, const float *inv_freq,
                          float *out, uint32_t ldo, float scale, hipStream_t stream);

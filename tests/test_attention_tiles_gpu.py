@@ -1,0 +1,92 @@
+"""mt_attention over many rows of one sequence (32-row blocks on the matrix cores) against the
+fp64 oracle and against the row kernels."""
+import numpy as np
+import pytest
+import torch
+
+import mingtts as mt
+import oracle as O
+from _gpu_util import say
+
+pytestmark = pytest.mark.gpu
+
+
+def _inputs(device, ct, M, hq, hkv, cap, seed, scale=1.5):
+    rng = np.random.default_rng(seed)
+    q = (rng.standard_normal((M, hq * 64)) * scale).astype(np.float32)
+    kc = torch.from_numpy(rng.standard_normal((hkv, cap, 64)).astype(np.float32)).to(device).to(ct)
+    vc = torch.from_numpy(rng.standard_normal((hkv, cap, 64)).astype(np.float32)).to(device).to(ct)
+    return q, kc, vc
+
+
+@pytest.mark.parametrize("ct,M,pos0,window,cap,hq,hkv", [
+    (torch.float16, 320, 0, 0, 320, 14, 2),       # the fewest rows without a window
+    (torch.float16, 333, 690, 0, 1024, 14, 2),    # a ragged last block, tiles cut by the block's end
+    (torch.float16, 65, 31, 65, 96, 14, 2),       # the fewest rows with one; the cache's last slot
+    (torch.float16, 97, 200, 1, 400, 3, 3),       # a window of the row itself
+    (torch.float32, 65, 192, 0, 257, 14, 2),      # the fewest keys of an fp32 cache without a window
+    (torch.float32, 130, 100, 65, 512, 4, 1),
+    (torch.float32, 70, 4026, 0, 4096, 2, 2),     # the longest cache
+])
+def test_tiles_match_fp64(gpu, ct, M, pos0, window, cap, hq, hkv):
+    """Sampled rows against fp64 on the stored cache values (the reference's tolerance, atol 2e-5 and
+    rtol 1e-4); cache rows no row attends hold NaN; a second run gives the same bits; out = q works."""
+    q, kc, vc = _inputs(gpu, ct, M, hq, hkv, cap, M * 5 + pos0 + window)
+    kg, vg = kc.double().cpu().numpy(), vc.double().cpu().numpy()
+    kc[:, pos0 + M:] = float("nan")
+    vc[:, pos0 + M:] = float("nan")
+    first = max(0, pos0 + 1 - window) if window else 0
+    kc[:, :first] = float("nan")
+    vc[:, :first] = float("nan")
+    qd = torch.from_numpy(q).to(gpu)
+    o = [torch.full((M, hq * 64), 7.0, device=gpu) for _ in range(2)]
+    say(f"attention tiles ct={ct} M={M} pos0={pos0} window={window} cap={cap} heads {hq}/{hkv}")
+    for out in o:
+        mt.attention(qd, hq * 64, M, hq, hkv, pos0, window, kc, vc, cap, out, hq * 64, 0.125)
+    mt.attention(qd, hq * 64, M, hq, hkv, pos0, window, kc, vc, cap, qd, hq * 64, 0.125)
+    torch.cuda.synchronize()
+    got = o[0].cpu().numpy()
+    np.testing.assert_array_equal(got, o[1].cpu().numpy())
+    np.testing.assert_array_equal(got, qd.cpu().numpy())
+    for m in sorted({0, 1, 31, 32, M // 2, M - 2, M - 1}):
+        want = O.attention_f64(q[m].reshape(hq, 64), kg, vg, pos0 + m, window, 0.125)
+        ex, i, g, w = O.worst_violation(got[m].reshape(hq, 64), want, 2e-5)
+        assert ex <= 0, f"row {m} index {i} got {g} want {w}"
+
+
+@pytest.mark.parametrize("ct", [torch.float16, torch.float32])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), float("-inf")])
+def test_values_that_are_not_finite_reach_only_the_rows_that_attend_them(gpu, ct, bad):
+    """A cached key or value, or a query, that is not finite: every row gets what the same row gets
+    from a call of its own (NaN in the same places), so rows before it stay finite."""
+    M, cap, at = 330, 512, 150
+    for where in ("k", "v", "q"):
+        q, kc, vc = _inputs(gpu, ct, M, 2, 1, cap, 11)
+        qd = torch.from_numpy(q).to(gpu)
+        (dict(k=kc, v=vc)[where][0, at] if where != "q" else qd[at])[5] = bad
+        o1 = torch.full((M, 128), 7.0, device=gpu)
+        o2 = torch.full((M, 128), 7.0, device=gpu)
+        say(f"attention tiles ct={ct} {bad} in {where}")
+        mt.attention(qd, 128, M, 2, 1, 0, 0, kc, vc, cap, o1, 128, 0.125)
+        for m in range(128, 192):
+            mt.attention(qd[m:], 128, 1, 2, 1, m, 0, kc, vc, cap, o2[m:], 128, 0.125)
+        torch.cuda.synchronize()
+        a, b = o1.cpu().numpy()[128:192], o2.cpu().numpy()[128:192]
+        assert np.isfinite(a[:at - 128]).all()
+        np.testing.assert_allclose(a, b, rtol=1e-4, atol=2e-5)
+
+
+def test_large_and_small_queries(gpu):
+    """The halves of q are scaled by the row's own power of two: queries of 1e-6 and of 1e5 (past
+    fp16's range), with a score scale that keeps the scores ordinary, and a negative scale."""
+    M, cap = 320, 320
+    for size, scale in ((1e-6, 1.2e5), (1e5, 1.2e-6), (1.0, -0.125)):
+        q, kc, vc = _inputs(gpu, torch.float16, M, 2, 1, cap, 3, size)
+        out = torch.full((M, 128), 7.0, device=gpu)
+        say(f"attention tiles q {size} scale {scale}")
+        mt.attention(torch.from_numpy(q).to(gpu), 128, M, 2, 1, 0, 0, kc, vc, cap, out, 128, scale)
+        torch.cuda.synchronize()
+        for m in (0, 100, M - 1):
+            want = O.attention_f64(q[m].reshape(2, 64), kc.double().cpu().numpy(), vc.double().cpu().numpy(), m, 0, scale)
+            ex, i, g, w = O.worst_violation(out[m].cpu().numpy().reshape(2, 64), want, 2e-5)
+            assert ex <= 0, f"row {m} index {i} got {g} want {w}"
