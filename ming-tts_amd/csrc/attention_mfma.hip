@@ -159,6 +159,7 @@ __global__ __launch_bounds__(AM_THREADS, 2) void attention_mfma_kernel(
                 for (int i = 0; i < 3; i++) qf[kk][i][e] = p[i];
             }
         }
+        tiled::settle<TY::MT>(qf[kk][1]);
     }
 
     f32x16t o[2];
@@ -279,6 +280,8 @@ __global__ __launch_bounds__(AM_THREADS, 2) void attention_mfma_kernel(
                     for (int i = 0; i < 3; i++) pf[kk][i][e] = w[i];
                 }
             }
+        tiled::settle<TY::MT>(pf[0][1]);
+        tiled::settle<TY::MT>(pf[1][1]);
 
         // p . v: d = 0 the even dims, 1 the odd ones.  A tile's sum starts from zero and joins the
         // running one in one rounding.

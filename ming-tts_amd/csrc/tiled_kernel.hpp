@@ -154,6 +154,15 @@ __device__ __forceinline__ void split8(const float (&x)[8], u32x4t &hi, u32x4t &
     }
 }
 
+// Between split8 and a VALU or MFMA instruction that reads lo: v_fma_mixhi moves its result to the
+// upper half of the register, and such a result takes one wait state before the next vector
+// instruction may read it.  The compiler inserts it for its own instructions, but does not look
+// into inline asm.  (Stores to LDS need none.)
+template <int T>
+__device__ __forceinline__ void settle(u32x4t &lo) {
+    if constexpr (T == DT_F16) asm("s_nop 0" : "+v"(lo));
+}
+
 template <int BM, int BN, bool GATED, int KS, bool SPLIT>
 struct TileShape {
     static constexpr int NW = 4 * KS;                 // waves: KS grids of 2 x 2 over the tile
