@@ -122,7 +122,9 @@ size_t tiled_partial_bytes(const TiledPlan &p, bool gated, bool norm) {
 //   M = 448-640 (204-255 tiles, 0.80-1)   17.4-19.5 / 28.9-30.8 against 19.8-21.0 / 35-36
 //   M = 704-768 (306 tiles, 0.60 of two)  32.3 / 54.6 against 21.9 / 45.3 (tiled)
 //   M = 1024 (408 tiles, 0.80 of two)     33.8 / 56.8 against 36.8 / 59.1
-// Below 384 rows (102 tiles or fewer) the tiled plans are faster as well.
+// Below 384 rows (102 tiles or fewer) the tiled plans are faster as well.  fp32 x of whole 64-k stages
+// takes the same tiles on the direct kernel (linear_gemm_direct.hip): 24.5 us at 512 rows, 47.9 at 1024;
+// ring_split_kernel keeps other K.
 static bool ring_fills(uint32_t M, uint32_t N, int cus) {
     const uint64_t t = static_cast<uint64_t>((M + ring::BM - 1) / ring::BM) * ((N + ring::FN - 1) / ring::FN);
     const uint64_t c = static_cast<uint64_t>(cus > 0 ? cus : 256);
@@ -137,6 +139,12 @@ int launch_gemm_tiled(const LinearArgs &a, int xt, int wt, hipStream_t stream, c
     const int cus = device_cus();
     if (cus <= 0) return set_error(MT_EHIP, "gemm: cannot query the device");
     const int tile = tuning().gemm_tile, splitk = tuning().gemm_splitk, stages_override = tuning().gemm_stages;
+    if (split && tile == 0 && splitk == 0 && stages_override == 0) {
+        const int d = direct_tile(a, cus, gated && ring_fills(a.M, a.N, cus));
+        if (d) return launch_gemm_direct(a, wt, d, stream);
+    }
+    // The gated 128 x 96 tiles by request: fp32 x on the direct kernel where it takes the linear.
+    if (split && gated && tile == 5 && direct_takes(a)) return launch_gemm_direct(a, wt, 2, stream);
     if (gated && !split && (tile == 5 || (tile == 0 && splitk == 0 && ring_fills(a.M, a.N, cus)))) {
         ring::RingArgs r{};
         r.x = static_cast<const uint16_t *>(a.x);

@@ -196,4 +196,10 @@ TiledPlan tiled_plan(uint32_t M, uint32_t N, uint32_t K, bool gated, int cus, in
 // x of the weights' type without a norm, or fp32 x with or without one (a.norm).
 int launch_gemm_tiled(const LinearArgs &a, int xt, int wt, hipStream_t stream, const FixedWs *fixed = nullptr);
 
+// The direct GEMM for fp32 x over many rows (direct_kernel.hpp): whether it can take a linear, the tile
+// it takes one in (0: it is left to tiled_plan's kernels), and its launch.
+bool direct_takes(const LinearArgs &a);
+int direct_tile(const LinearArgs &a, int cus, bool ring_fills);
+int launch_gemm_direct(const LinearArgs &a, int wt, int tile, hipStream_t stream);
+
 }  // namespace mt

@@ -1,0 +1,59 @@
+"""The direct GEMM for fp32 x over many rows (mt_linear / mt_linear_rmsnorm): each of its tiles at the
+sizes where the choice takes it, against fp64."""
+import numpy as np
+import pytest
+import torch
+
+import mingtts as mt
+import oracle as O
+from _gpu_util import say
+
+pytestmark = pytest.mark.gpu
+
+# M, N, K, gated, norm: 64 x 96 features (gated), 128 x 96 (gated, and one past its last wave), 64 x
+# 192, 128 x 192 and 128 x 128 weight rows, with ragged rows and features; odd and even stage counts
+# (8, 14, 15, 31); the shortest and the longest K.
+CASES = [(257, 4864, 896, True, True), (330, 4800, 512, True, False), (513, 4850, 896, True, True), (1793, 1152, 896, False, True),
+         (1601, 3072, 1024, False, True), (900, 4096, 1024, False, True), (1100, 4099, 512, False, False),
+         (2047, 1031, 1984, False, False), (1300, 4099, 960, False, True)]
+
+
+@pytest.mark.parametrize("wt", [O.F16, O.BF16], ids=["wf16", "wbf16"])
+@pytest.mark.parametrize("M,N,K,gated,norm", CASES)
+def test_direct_gemm_matches_fp64(gpu, M, N, K, gated, norm, wt):
+    """x in a wider matrix (ldx > K) with NaN between its rows, y in a wider one that keeps what lies
+    between, bias and accumulate; normwise within the bound of x in two halves (2^-22 of x with fp16,
+    2^-17 with bf16) plus fp32 sums, and twice the same bits."""
+    say(f"direct gemm {M}x{N}x{K} gated={gated} norm={norm} w{wt}")
+    dt = torch.float16 if wt == O.F16 else torch.bfloat16
+    g = torch.Generator(device=gpu)
+    g.manual_seed(M + N + K)
+    rand = lambda *s, sc=1.0: torch.randn(*s, generator=g, device=gpu) * sc  # noqa: E731
+    ldx, ldy = K + 8, N + 5
+    xs = torch.full((M, ldx), float("nan"), device=gpu)
+    xs[:, :K] = rand(M, K)
+    w, w2 = rand(N, K, sc=0.02).to(dt), rand(N, K, sc=0.02).to(dt)
+    b, gain = rand(N, sc=0.1).to(dt), (1.0 + 0.1 * rand(K)).to(dt)
+    y0 = rand(M, ldy)
+    flags = mt.GemvFlags.accumulate | (mt.GemvFlags.siluGate if gated else 0)
+    runs = []
+    for _ in range(2):
+        y = y0.clone()
+        mt.linear(xs, w, y, flags=flags, w2=w2 if gated else None, bias=b, ldx=ldx, ldy=ldy, norm=gain if norm else None)
+        torch.cuda.synchronize()
+        runs.append(y)
+    assert torch.equal(runs[0], runs[1])
+    assert torch.equal(runs[0][:, N:], y0[:, N:])
+    x = xs[:, :K].double()
+    if norm:
+        x = x * torch.rsqrt((x * x).mean(-1, keepdim=True) + 1e-6) * gain.double()
+    v = x @ w.double().t().contiguous() + b.double()
+    if gated:
+        v = v / (1.0 + torch.exp(-v)) * (x @ w2.double().t().contiguous())
+    want = y0[:, :N].double() + v
+    got = runs[0][:, :N].double()
+    # halves: 2^-22 / 2^-17 of each product; sums: K / 16 roundings of 2^-24 each way
+    bound = (2.0 ** -22 if wt == O.F16 else 2.0 ** -17) + 2.0 ** -24 * (K / 16) ** 0.5
+    assert ((got - want).norm() / want.norm()).item() <= 2 * bound
+    scale = v.pow(2).mean().sqrt()
+    assert ((got - want).abs().max() / scale).item() <= 40 * bound
