@@ -13,8 +13,8 @@
 //   - p.v: 16 lanes cover the 64 dims of one V row (4 dims each, one coalesced row per
 //     16 lanes), 16 key phases per workgroup, 32 rows per lane requested at a time,
 //     partial sums meet in LDS in a fixed order.
-// Batched decode (mt_attention_decode) is the same kernel with a per-row cache base and
-// the row's query position read from a device array.
+// Batched decode (mt_attention_decode, a cache and a device-side length per row) has a kernel of
+// its own, and many rows of one sequence go to the matrix cores (attention_mfma.hip).
 #include "attend_row.hpp"
 #include "mt_device.hpp"
 #include "mt_internal.hpp"
@@ -86,25 +86,136 @@ __global__ __launch_bounds__(256) void rope_cache_kernel(float *qkv, uint32_t ld
 }
 
 template <int CT>
-__global__ __launch_bounds__(ATT_THREADS) void attention_kernel(const float *q, uint32_t ldq, uint32_t hq,
-                                                                uint32_t hkv, uint32_t pos0, const uint32_t *lens,
-                                                                uint32_t window, const void *kc, const void *vc,
-                                                                uint32_t cache_len, uint64_t cache_stride,
-                                                                float *out, uint32_t ldo, float scale) {
+__global__ __launch_bounds__(ATT_THREADS) void attention_kernel(const float *q, uint32_t ldq, uint32_t hq, uint32_t hkv,
+                                                                uint32_t pos0, uint32_t window, const void *kc,
+                                                                const void *vc, uint32_t cache_len, float *out,
+                                                                uint32_t ldo, float scale) {
     __shared__ RowLds lds;
     const uint32_t m = blockIdx.x / hq, h = blockIdx.x % hq;
     const uint32_t kvh = h / (hq / hkv);
-    // Device-side lengths are clamped to the cache; a zero length attends to nothing and
-    // writes zeros.
-    const uint32_t len = lens ? min(lens[m], cache_len) : pos0 + m + 1;
-    const uint64_t cbase = lens ? static_cast<uint64_t>(m) * cache_stride : 0;
-    const uint32_t jEnd = len;
+    const uint32_t jEnd = pos0 + m + 1;
+    const uint32_t jStart = (window > 0 && jEnd > window) ? jEnd - window : 0;
+    attend_row<CT, 16, 32>(q + static_cast<size_t>(m) * ldq + h * 64, kc, vc,
+                           (static_cast<size_t>(kvh) * cache_len + jStart) * 64, static_cast<int>(jEnd - jStart), scale,
+                           out + static_cast<size_t>(m) * ldo + h * 64, lds.sc, lds.red, lds.part);
+}
+
+// A decode row's attention: one 1024-thread workgroup per (row, head).  An octet of lanes owns keys
+// kq, kq + 128, ... and lane r of it dims 8r .. 8r + 7 of both k and v, so a round's keys and values (KU
+// of each an octet) are requested together and one round trip to memory serves the scores and p.v.
+// A wave's octets share a running maximum; their sums meet by lane exchanges inside the wave and the
+// waves' through LDS, in a fixed order (a maximum for the whole workgroup, one barrier a round, was no
+// more exact and took 0.8 us more).  The row kernel (four waves, the values requested after the softmax)
+// waits for twice the round trips with a quarter of the loads in flight.  Graph replay, 14 / 2 heads,
+// lengths up to the cache's, fp16 / fp32 cache: eight sequences of up to 2048 keys 19.2 / 23.1 -> 9.4
+// / 16.4 us, of up to 512 6.7 / 7.1 -> 5.7 / 5.4, one of up to 2048 18.1 / 20.1 -> 8.1 / 11.0.
+constexpr int WD_THREADS = 1024, WD_WAVES = WD_THREADS / 64, WD_KP = WD_THREADS / 8;
+template <int CT>
+__global__ __launch_bounds__(WD_THREADS) void attention_decode_kernel(const float *q, uint32_t ldq, uint32_t hq, uint32_t hkv,
+                                                                      const uint32_t *lens, uint32_t window, const void *kc,
+                                                                      const void *vc, uint32_t cache_len,
+                                                                      uint64_t cache_stride, float *out, uint32_t ldo,
+                                                                      float scale) {
+    constexpr int KU = CT == DT_F32 ? 4 : 8;  // keys an octet requests at a time
+    __shared__ float wm[WD_WAVES], wl[WD_WAVES];
+    __shared__ __attribute__((aligned(16))) float wo[WD_WAVES][64];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const uint32_t m = blockIdx.x / hq, h = blockIdx.x % hq, kvh = h / (hq / hkv);
+    // Device-side lengths are clamped to the cache; a zero length attends to nothing and writes
+    // zeros.
+    const uint32_t jEnd = min(lens[m], cache_len);
     const uint32_t jStart = (window > 0 && jEnd > window) ? jEnd - window : 0;
     const int nk = static_cast<int>(jEnd - jStart);
-    const size_t kvbase = cbase + (static_cast<size_t>(kvh) * cache_len + jStart) * 64;
-
-    attend_row<CT, 16, 32>(q + static_cast<size_t>(m) * ldq + h * 64, kc, vc, kvbase, nk, scale,
-                           out + static_cast<size_t>(m) * ldo + h * 64, lds.sc, lds.red, lds.part);
+    const int r = tid & 7, kq = tid >> 3;
+    const size_t base = static_cast<uint64_t>(m) * cache_stride + (static_cast<size_t>(kvh) * cache_len + jStart) * 64 + 8 * r;
+    float qf[8];
+    {
+        const float4 *qp = reinterpret_cast<const float4 *>(q + static_cast<size_t>(m) * ldq + h * 64 + 8 * r);
+        const float4 a = qp[0], b = qp[1];
+        qf[0] = a.x; qf[1] = a.y; qf[2] = a.z; qf[3] = a.w;
+        qf[4] = b.x; qf[5] = b.y; qf[6] = b.z; qf[7] = b.w;
+    }
+    float mx = -INFINITY, l = 0.0f, acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    for (int j0 = 0; j0 < nk; j0 += KU * WD_KP) {
+        const int t0 = j0 + kq;
+        // Keys past the end re-read the last one and are skipped.
+        Raw8<CT> kr[KU], vr[KU];
+#pragma unroll
+        for (int u = 0; u < KU; u++) kr[u] = load8_raw<CT>(kc, base + static_cast<size_t>(min(t0 + u * WD_KP, nk - 1)) * 64);
+#pragma unroll
+        for (int u = 0; u < KU; u++) vr[u] = load8_raw<CT>(vc, base + static_cast<size_t>(min(t0 + u * WD_KP, nk - 1)) * 64);
+        __builtin_amdgcn_sched_barrier(0);  // every request ahead of the first use
+        float s[KU], mn = mx;
+#pragma unroll
+        for (int u = 0; u < KU; u++) {
+            float kf[8], v = 0.0f;
+            decode8<CT>(kr[u], kf);
+#pragma unroll
+            for (int e = 0; e < 8; e++) v = fmaf(qf[e], kf[e], v);
+            s[u] = v;
+        }
+        octet_sums<KU>(s);
+#pragma unroll
+        for (int u = 0; u < KU; u++) {
+            s[u] *= scale;
+            if (t0 + u * WD_KP < nk) mn = fmaxf(mn, s[u]);
+        }
+        mn = wave_max(mn);
+        const float al = mn == mx ? 1.0f : exp_hw(mx - mn), ms = mn == -INFINITY ? 0.0f : mn;
+        mx = mn;
+        l *= al;
+#pragma unroll
+        for (int e = 0; e < 8; e++) acc[e] *= al;
+#pragma unroll
+        for (int u = 0; u < KU; u++) {
+            if (t0 + u * WD_KP < nk) {  // the 8 lanes of a key agree
+                const float p = exp_hw(s[u] - ms);
+                float vf[8];
+                decode8<CT>(vr[u], vf);
+                l += p;
+#pragma unroll
+                for (int e = 0; e < 8; e++) acc[e] = fmaf(p, vf[e], acc[e]);
+            }
+        }
+    }
+    // The wave's eight octets: lanes r, r + 8, ... hold the same dims of different keys.
+#pragma unroll
+    for (int d = 8; d < 64; d <<= 1) {
+        l += __shfl_xor(l, d, 64);
+#pragma unroll
+        for (int e = 0; e < 8; e++) acc[e] += __shfl_xor(acc[e], d, 64);
+    }
+    if (lane < 8) {
+        *reinterpret_cast<float4 *>(&wo[wave][8 * lane]) = make_float4(acc[0], acc[1], acc[2], acc[3]);
+        *reinterpret_cast<float4 *>(&wo[wave][8 * lane + 4]) = make_float4(acc[4], acc[5], acc[6], acc[7]);
+        if (lane == 0) {
+            wm[wave] = mx;
+            wl[wave] = l;
+        }
+    }
+    __syncthreads();
+    if (tid < 64) {
+        float mm = wm[0], o[WD_WAVES], g[WD_WAVES];
+#pragma unroll
+        for (int w = 1; w < WD_WAVES; w++) mm = fmaxf(mm, wm[w]);
+#pragma unroll
+        for (int w = 0; w < WD_WAVES; w++) {
+            const float f = wm[w] == mm ? 1.0f : exp_hw(wm[w] - mm);  // 0 for a wave without keys
+            g[w] = wl[w] * f;
+            o[w] = wo[w][tid] * f;
+        }
+#pragma unroll
+        for (int d = WD_WAVES / 2; d > 0; d >>= 1)
+#pragma unroll
+            for (int w = 0; w < d; w++) {
+                g[w] += g[w + d];
+                o[w] += o[w + d];
+            }
+        const float sum = g[0];
+        // No key: zeros.  Keys whose scores are all -infinity have no softmax.
+        const float inv = sum > 0.0f ? 1.0f / sum : nk > 0 ? NAN : 0.0f;
+        out[static_cast<size_t>(m) * ldo + h * 64 + tid] = o[0] * inv;
+    }
 }
 
 // attention_kernel's arithmetic for R consecutive rows of one sequence at a time, for rows whose
@@ -553,10 +664,20 @@ int launch_attention(const float *q, uint32_t ldq, uint32_t rows, uint32_t hq, u
                      const uint32_t *lens, uint32_t window, const void *kc, const void *vc, int ct,
                      uint32_t cache_len, uint64_t cache_stride, float *out, uint32_t ldo, float scale,
                      hipStream_t stream) {
-    if (!lens && attention_tiles(rows, pos0, window, ct))
+    if (lens) {
+        const dim3 g(rows * hq);
+        if (ct == DT_F32)
+            hipLaunchKernelGGL(attention_decode_kernel<DT_F32>, g, dim3(WD_THREADS), 0, stream, q, ldq, hq, hkv, lens, window,
+                               kc, vc, cache_len, cache_stride, out, ldo, scale);
+        else
+            hipLaunchKernelGGL(attention_decode_kernel<DT_F16>, g, dim3(WD_THREADS), 0, stream, q, ldq, hq, hkv, lens, window,
+                               kc, vc, cache_len, cache_stride, out, ldo, scale);
+        return check_launch("attention (decode)");
+    }
+    if (attention_tiles(rows, pos0, window, ct))
         return launch_attention_mfma(q, ldq, rows, hq, hkv, pos0, window, kc, vc, ct, cache_len, out, ldo, scale, stream);
     // Rows of one sequence whose keys all start at position 0 go by blocks of AR_ROWS rows.
-    if (!lens && rows >= AR_MIN_ROWS && pos0 + rows <= static_cast<uint32_t>(AR_MAXKEYS) &&
+    if (rows >= AR_MIN_ROWS && pos0 + rows <= static_cast<uint32_t>(AR_MAXKEYS) &&
         (window == 0 || pos0 + rows <= window)) {
         const dim3 g(hq, (rows + AR_ROWS - 1) / AR_ROWS);
         if (ct == DT_F32)
@@ -569,11 +690,11 @@ int launch_attention(const float *q, uint32_t ldq, uint32_t rows, uint32_t hq, u
     }
     dim3 grid(rows * hq);
     if (ct == DT_F32)
-        hipLaunchKernelGGL(attention_kernel<DT_F32>, grid, dim3(ATT_THREADS), 0, stream, q, ldq, hq, hkv, pos0, lens,
-                           window, kc, vc, cache_len, cache_stride, out, ldo, scale);
+        hipLaunchKernelGGL(attention_kernel<DT_F32>, grid, dim3(ATT_THREADS), 0, stream, q, ldq, hq, hkv, pos0, window,
+                           kc, vc, cache_len, out, ldo, scale);
     else
-        hipLaunchKernelGGL(attention_kernel<DT_F16>, grid, dim3(ATT_THREADS), 0, stream, q, ldq, hq, hkv, pos0, lens,
-                           window, kc, vc, cache_len, cache_stride, out, ldo, scale);
+        hipLaunchKernelGGL(attention_kernel<DT_F16>, grid, dim3(ATT_THREADS), 0, stream, q, ldq, hq, hkv, pos0, window,
+                           kc, vc, cache_len, out, ldo, scale);
     return check_launch("attention");
 }
 

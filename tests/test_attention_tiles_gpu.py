@@ -90,3 +90,31 @@ def test_large_and_small_queries(gpu):
             want = O.attention_f64(q[m].reshape(2, 64), kc.double().cpu().numpy(), vc.double().cpu().numpy(), m, 0, scale)
             ex, i, g, w = O.worst_violation(out[m].cpu().numpy().reshape(2, 64), want, 2e-5)
             assert ex <= 0, f"row {m} index {i} got {g} want {w}"
+
+
+@pytest.mark.parametrize("ct,cap", [(torch.float32, 1600), (torch.float16, 2100), (torch.float16, 40)])
+def test_decode_rounds_match_fp64(gpu, ct, cap):
+    """mt_attention_decode at the edges of its rounds (512 keys of an fp32 cache, 1024 of an fp16 one) and
+    of its octets, NaN in the cache rows past each length, a maximum that moves in the last round, and
+    more query heads than a wave has octets."""
+    lens = np.array([n for n in (1, 7, 9, 128, 129, 511, 512, 513, 1023, 1024, 1025, cap) if n <= cap], np.uint32)
+    B, hq, hkv = len(lens), 14, 2
+    rng = np.random.default_rng(cap)
+    q = (rng.standard_normal((B, hq * 64)) * 1.5).astype(np.float32)
+    kc = torch.from_numpy(rng.standard_normal((B, hkv, cap, 64)).astype(np.float32)).to(gpu).to(ct)
+    vc = torch.from_numpy(rng.standard_normal((B, hkv, cap, 64)).astype(np.float32)).to(gpu).to(ct)
+    for b, n in enumerate(lens):
+        kc[b, 0, int(n) - 1] *= 4.0
+        kc[b, :, int(n):] = float("nan")
+        vc[b, :, int(n):] = float("nan")
+    out = torch.full((B, hq * 64), 7.0, device=gpu)
+    say(f"decode rounds ct={ct} cap={cap} lens={lens.tolist()}")
+    mt.attention_decode(torch.from_numpy(q).to(gpu), hq * 64, B, hq, hkv, torch.from_numpy(lens.astype(np.int32)).to(gpu), 0,
+                        kc, vc, cap, hkv * cap * 64, out, hq * 64, 0.125)
+    torch.cuda.synchronize()
+    got = out.cpu().numpy().reshape(B, hq, 64)
+    for b, n in enumerate(lens):
+        want = O.attention_f64(q[b].reshape(hq, 64), kc[b].double().cpu().numpy(), vc[b].double().cpu().numpy(), int(n) - 1, 0,
+                               0.125)
+        ex, i, g, w = O.worst_violation(got[b], want, 2e-5)
+        assert ex <= 0, f"len {n} index {i} got {g} want {w}"
