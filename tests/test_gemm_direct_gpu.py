@@ -15,7 +15,10 @@ pytestmark = pytest.mark.gpu
 # (8, 14, 15, 31); the shortest and the longest K.
 CASES = [(257, 4864, 896, True, True), (330, 4800, 512, True, False), (513, 4850, 896, True, True), (1793, 1152, 896, False, True),
          (1601, 3072, 1024, False, True), (900, 4096, 1024, False, True), (1100, 4099, 512, False, False),
-         (2047, 1031, 1984, False, False), (1300, 4099, 960, False, True)]
+         (2047, 1031, 1984, False, False), (1300, 4099, 960, False, True),
+         # long K: three parts, two, and parts of unequal length with ragged tiles
+         (1024, 896, 4864, False, False), (1601, 890, 4864, False, False),
+         (1100, 1000, 2112, False, False)]
 
 
 @pytest.mark.parametrize("wt", [O.F16, O.BF16], ids=["wf16", "wbf16"])
@@ -57,3 +60,27 @@ def test_direct_gemm_matches_fp64(gpu, M, N, K, gated, norm, wt):
     assert ((got - want).norm() / want.norm()).item() <= 2 * bound
     scale = v.pow(2).mean().sqrt()
     assert ((got - want).abs().max() / scale).item() <= 40 * bound
+
+
+def test_long_k_under_capture_without_a_workspace(gpu):
+    """A stream captured before its workspace exists takes the linear all the same (on the kernel that
+    needs none), and every replay gives the eager bits of that kernel's tolerance."""
+    M, N, K = 1600, 896, 4864
+    say("direct gemm: long K under capture")
+    g = torch.Generator(device=gpu)
+    g.manual_seed(9)
+    x = torch.randn(M, K, generator=g, device=gpu)
+    w = (torch.randn(N, K, generator=g, device=gpu) * 0.02).half()
+    want = x.double() @ w.double().t().contiguous()
+    y = torch.zeros(M, N, device=gpu)
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        mt.linear(x, w, y, stream=s)
+    for _ in range(3):
+        y.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert ((y.double() - want).norm() / want.norm()).item() <= 2e-6
