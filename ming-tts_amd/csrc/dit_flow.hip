@@ -119,8 +119,13 @@ __global__ __launch_bounds__(256) void flow_euler_kernel(float *y, const float *
 // of the latent in place (kept in LDS), then the six flow-input rows, thread c taking column
 // c; rows 1 and 4 (x_b + x_w history) and rows 2 and 5 (x_b + x_w y) are the same sums, so
 // each is computed once and stored twice.  Same arithmetic as the two kernels.
+//
+// ROWS64 (latent 64, hidden up to 1024: the flow head's): a thread's embedder row is 128 bytes of its
+// own, so loading it straight takes a cycle for each of a wave's 64 rows and each of its 8 chunks,
+// 3.4 us of the one CU this runs on.  The rows are loaded in order instead (eight threads a row) and
+// pass through LDS, chunk c of row r in slot c ^ (r & 7): 6.05 -> 4.28 us a launch (graph replay), the same sums.
 constexpr uint32_t FLOW_LATENT_MAX = 2048;
-template <int WT>
+template <int WT, bool ROWS64>
 __global__ __launch_bounds__(1024) void flow_euler_assemble_kernel(float *y, const float *pred, uint32_t ldp,
                                                                   uint32_t pred_row, uint32_t null_row, float *capture,
                                                                   float cfg, float dt, const float *history,
@@ -128,12 +133,20 @@ __global__ __launch_bounds__(1024) void flow_euler_assemble_kernel(float *y, con
                                                                   const float *temb, const uint16_t *xw,
                                                                   const uint16_t *xb, float *x, uint32_t ldx,
                                                                   uint32_t hidden, uint32_t latent) {
-    __shared__ float ys[FLOW_LATENT_MAX], hs[FLOW_LATENT_MAX];
+    constexpr uint32_t LMAX = ROWS64 ? 64 : FLOW_LATENT_MAX;
+    __shared__ float ys[LMAX], hs[LMAX];
+    __shared__ uint4 rows[ROWS64 ? 1024 * EMB_CHUNKS : 1];
     // The inputs of this thread's first column (clamped into the matrix: hidden >= 1) are
     // requested before the Euler update, so their round trip overlaps the update's.
     uint32_t c = min(threadIdx.x, hidden - 1);
     uint4 wv[EMB_CHUNKS];
-    emb_chunks(xw + static_cast<size_t>(c) * latent, 0, latent, wv);
+    if constexpr (ROWS64) {  // chunk threadIdx.x % 8 of rows threadIdx.x / 8 + 128 i
+#pragma unroll
+        for (uint32_t i = 0; i < EMB_CHUNKS; i++)
+            wv[i] = reinterpret_cast<const uint4 *>(xw)[min(threadIdx.x + 1024 * i, hidden * 8 - 1)];
+    } else {
+        emb_chunks(xw + static_cast<size_t>(c) * latent, 0, latent, wv);
+    }
     float te = temb[c], ce = cemb[c];
     uint16_t cb = cbias[c], bb = xb[c];
     for (uint32_t d = threadIdx.x; d < latent; d += blockDim.x) {
@@ -148,7 +161,16 @@ __global__ __launch_bounds__(1024) void flow_euler_assemble_kernel(float *y, con
         ys[d] = v;
         hs[d] = history[d];
     }
+    if constexpr (ROWS64) {
+        const uint32_t r = threadIdx.x >> 3, k = threadIdx.x & 7;
+#pragma unroll
+        for (uint32_t i = 0; i < EMB_CHUNKS; i++) rows[(r + 128 * i) * 8 + (k ^ (r & 7))] = wv[i];
+    }
     __syncthreads();
+    if constexpr (ROWS64) {
+#pragma unroll
+        for (uint32_t i = 0; i < EMB_CHUNKS; i++) wv[i] = rows[c * 8 + (i ^ (c & 7))];
+    }
     // Column c's six rows, the first batch of its embedder row's chunks in w0.
     const auto column = [&](uint32_t c, const uint4 (&w0)[EMB_CHUNKS], float te, float ce, uint16_t cb, uint16_t bb,
                             uint32_t z) {
@@ -202,12 +224,12 @@ int launch_flow_euler_assemble(float *y, const float *pred, uint32_t ldp, uint32
                                uint32_t ldx, uint32_t hidden, uint32_t latent, hipStream_t stream) {
     const uint16_t *cb = static_cast<const uint16_t *>(cbias), *w = static_cast<const uint16_t *>(xw),
                    *b = static_cast<const uint16_t *>(xb);
-    if (wt == DT_BF16)
-        hipLaunchKernelGGL(flow_euler_assemble_kernel<DT_BF16>, dim3(1), dim3(1024), 0, stream, y, pred, ldp, pred_row,
-                           null_row, capture, cfg, dt, history, cemb, cb, temb, w, b, x, ldx, hidden, latent);
-    else
-        hipLaunchKernelGGL(flow_euler_assemble_kernel<DT_F16>, dim3(1), dim3(1024), 0, stream, y, pred, ldp, pred_row,
-                           null_row, capture, cfg, dt, history, cemb, cb, temb, w, b, x, ldx, hidden, latent);
+    const bool rows64 = latent == 64 && hidden <= 1024;
+    const auto kernel = wt == DT_BF16
+                            ? (rows64 ? flow_euler_assemble_kernel<DT_BF16, true> : flow_euler_assemble_kernel<DT_BF16, false>)
+                            : (rows64 ? flow_euler_assemble_kernel<DT_F16, true> : flow_euler_assemble_kernel<DT_F16, false>);
+    hipLaunchKernelGGL(kernel, dim3(1), dim3(1024), 0, stream, y, pred, ldp, pred_row, null_row, capture, cfg, dt, history,
+                       cemb, cb, temb, w, b, x, ldx, hidden, latent);
     return check_launch("flow_euler_assemble");
 }
 
