@@ -70,7 +70,11 @@ bool workspace_ready(const FixedWs *fixed, hipStream_t stream, size_t part_bytes
         if (it != g_ws.end() && it->second.base && it->second.part_bytes >= part_bytes) return true;
     }
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    return hipStreamIsCapturing(stream, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &cs) != hipSuccess) {  // e.g. the legacy stream beside a global capture
+        (void)hipGetLastError();  // not the launch's error
+        return false;
+    }
+    return cs == hipStreamCaptureStatusNone;
 }
 
 int stream_workspace(hipStream_t stream, size_t part_bytes, uint32_t counters, void **part, uint32_t **cnt) {
