@@ -181,7 +181,8 @@ enum {
                                     gated ring kernel (128 x rows x 96 features of W and W2; SiLU-gated
                                     linears only: the auto choice when its tiles fill at least
                                     3/4 of their last wave on the CUs, e.g. gate|up at 448-640
-                                    rows on 256 CUs) */
+                                    rows on 256 CUs; fp32 x of whole 64-k stages takes
+                                    these tiles on the direct kernel) */
     MT_TUNE_GEMM_STAGES = 7,     /* loads of that GEMM for x of the weights' type: 2..4 = direct-to-LDS
                                     stages of 64 k, 1 = two register-staged stages into two LDS
                                     buffers (0 = auto); fp32 x always stages through registers,
