@@ -364,7 +364,9 @@ int mt_rope_cache_decode(float *qkv, uint32_t ldq, uint32_t B, uint32_t hq, uint
  * max-subtracted softmax, out = sum p v.  q rows hold hq heads of 64 (stride ldq),
  * out rows stride ldo.  pos0 + M <= cache_len <= 4096.  Rows of a prefill (M >= 8, every
  * row's keys starting at 0, pos0 + M <= 1024) are attended 4 to a workgroup; the results
- * are bit-identical to attending the rows one call each.
+ * are bit-identical to attending the rows one call each.  So are up to 64 rows of any other
+ * call; more of them (keys past 1024, or a window that cuts them) run on the matrix cores, whose
+ * sums are of another order.
  */
 int mt_attention(const float *q, uint32_t ldq, uint32_t M, uint32_t hq, uint32_t hkv,
                  uint32_t pos0, uint32_t window, const void *k_cache, const void *v_cache,

@@ -647,17 +647,22 @@ int launch_rope_cache(float *qkv, uint32_t ldq, uint32_t rows, uint32_t hq, uint
     return check_launch("rope_cache");
 }
 
-// Rows of one sequence that go by 32-row blocks on the matrix cores (attention_mfma.hip).  Up to
-// 64 rows (mt_rope_attention's range) and, without a window, up to 256 keys or 320 fp16 rows the
-// row kernels are kept: there their results are those of the rows attended one call each, bit for
-// bit, and with an fp32 cache they are as fast (174 rows 7.6 against 7.7 us).  Above, graph replay,
-// row kernels against the matrix cores, fp16 / fp32 cache: 512 rows 21.4 / 21.2 against 7.4 / 11.7
-// us, 2048 rows 431 / 766 against 31 / 64 us, window 65: 100 rows 12.2 / 17.4 against 4.7 / 5.5
-// us, 1600 rows 132 / 233 against 10.1 / 12.4 us.
-static bool attention_tiles(uint32_t rows, uint32_t pos0, uint32_t window, int ct) {
-    if (rows <= 64) return false;
-    if (window > 0 && pos0 + rows > window) return true;
-    return ct == DT_F32 ? pos0 + rows > 256 : rows >= 320;
+// Do every row's keys start at position 0 and end by AR_MAXKEYS?  Such rows give the bits of one call
+// each (mt_attention's contract), so they stay on the row kernel's arithmetic whatever their number,
+// by blocks of AR_ROWS rows from AR_MIN_ROWS rows on.
+static bool row_blocks(uint32_t rows, uint32_t pos0, uint32_t window) {
+    return pos0 + rows <= static_cast<uint32_t>(AR_MAXKEYS) && (window == 0 || pos0 + rows <= window);
+}
+
+// The others go by 32-row blocks on the matrix cores (attention_mfma.hip) above 64 rows; up to there
+// mt_rope_attention gives mt_attention's bits, so both run the row kernel.  Graph replay, row kernel
+// against the matrix cores, fp16 / fp32 cache, 14 / 2 heads: 65 rows after 1024 keys 24.9 / 35.3
+// against 10.7 / 19.8 us, 301 rows after 1024 84 / 138 against 12.5 / 24.2, 2048 rows from 0 432 / 771
+// against 31.8 / 65.4; window 65: 65 rows 9.7 / 12.7 against 4.8 / 6.0, 1600 rows 132 / 234 against 10.2 /
+// 12.8.  Within 1024 keys the contract costs speed: 512 rows 21.5 / 21.3 us by blocks of rows, 7.4 / 11.7
+// on the matrix cores.
+static bool attention_tiles(uint32_t rows, uint32_t pos0, uint32_t window) {
+    return rows > 64 && !row_blocks(rows, pos0, window);
 }
 
 int launch_attention(const float *q, uint32_t ldq, uint32_t rows, uint32_t hq, uint32_t hkv, uint32_t pos0,
@@ -674,11 +679,9 @@ int launch_attention(const float *q, uint32_t ldq, uint32_t rows, uint32_t hq, u
                                kc, vc, cache_len, cache_stride, out, ldo, scale);
         return check_launch("attention (decode)");
     }
-    if (attention_tiles(rows, pos0, window, ct))
+    if (attention_tiles(rows, pos0, window))
         return launch_attention_mfma(q, ldq, rows, hq, hkv, pos0, window, kc, vc, ct, cache_len, out, ldo, scale, stream);
-    // Rows of one sequence whose keys all start at position 0 go by blocks of AR_ROWS rows.
-    if (rows >= AR_MIN_ROWS && pos0 + rows <= static_cast<uint32_t>(AR_MAXKEYS) &&
-        (window == 0 || pos0 + rows <= window)) {
+    if (rows >= AR_MIN_ROWS && row_blocks(rows, pos0, window)) {
         const dim3 g(hq, (rows + AR_ROWS - 1) / AR_ROWS);
         if (ct == DT_F32)
             hipLaunchKernelGGL((attention_rows_kernel<DT_F32, AR_ROWS>), g, dim3(ATT_THREADS), 0, stream, q, ldq, hq,

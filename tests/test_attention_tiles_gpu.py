@@ -19,18 +19,50 @@ def _inputs(device, ct, M, hq, hkv, cap, seed, scale=1.5):
     return q, kc, vc
 
 
+def _tiles(M, pos0, window):
+    """Whether mt_attention takes the matrix cores: more than 64 rows, unless every row's keys start at
+    position 0 and end by 1024 (those keep the bits of one call per row)."""
+    return M > 64 and not (pos0 + M <= 1024 and (window == 0 or pos0 + M <= window))
+
+
+@pytest.mark.parametrize("ct,M,pos0,window", [
+    (torch.float16, 320, 0, 0),
+    (torch.float16, 1024, 0, 0),     # the last key within the contract
+    (torch.float16, 500, 524, 0),
+    (torch.float16, 400, 0, 400),    # a window as long as the last row's span
+    (torch.float32, 65, 192, 0),
+    (torch.float32, 512, 0, 0),
+    (torch.float32, 700, 324, 0),
+])
+def test_rows_within_1024_keys_have_the_bits_of_one_call_each(gpu, ct, M, pos0, window):
+    """mt_attention's contract for M >= 8 rows whose keys start at position 0 and end by 1024, at row
+    counts and spans where the matrix cores would take the rows otherwise."""
+    assert not _tiles(M, pos0, window)
+    q, kc, vc = _inputs(gpu, ct, M, 2, 1, 1024, M + pos0)
+    qd = torch.from_numpy(q).to(gpu)
+    o1, o2 = torch.full((M, 128), 7.0, device=gpu), torch.full((M, 128), 7.0, device=gpu)
+    say(f"rows within 1024 keys ct={ct} M={M} pos0={pos0} window={window}")
+    mt.attention(qd, 128, M, 2, 1, pos0, window, kc, vc, 1024, o1, 128, 0.125)
+    for m in range(M):
+        mt.attention(qd[m:], 128, 1, 2, 1, pos0 + m, window, kc, vc, 1024, o2[m:], 128, 0.125)
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(o1.cpu().numpy(), o2.cpu().numpy())
+
+
 @pytest.mark.parametrize("ct,M,pos0,window,cap,hq,hkv", [
-    (torch.float16, 320, 0, 0, 320, 14, 2),       # the fewest rows without a window
-    (torch.float16, 333, 690, 0, 1024, 14, 2),    # a ragged last block, tiles cut by the block's end
-    (torch.float16, 65, 31, 65, 96, 14, 2),       # the fewest rows with one; the cache's last slot
+    (torch.float16, 65, 960, 0, 1025, 14, 2),     # the fewest rows, one key past the row kernels' 1024
+    (torch.float16, 333, 800, 0, 1136, 14, 2),    # a ragged last block, tiles cut by the block's end
+    (torch.float16, 65, 31, 65, 96, 14, 2),       # the fewest rows with a window; the cache's last slot
     (torch.float16, 97, 200, 1, 400, 3, 3),       # a window of the row itself
-    (torch.float32, 65, 192, 0, 257, 14, 2),      # the fewest keys of an fp32 cache without a window
+    (torch.float16, 81, 0, 80, 81, 14, 2),        # a window that cuts the last row alone
+    (torch.float32, 65, 960, 0, 1025, 14, 2),
     (torch.float32, 130, 100, 65, 512, 4, 1),
     (torch.float32, 70, 4026, 0, 4096, 2, 2),     # the longest cache
 ])
 def test_tiles_match_fp64(gpu, ct, M, pos0, window, cap, hq, hkv):
     """Sampled rows against fp64 on the stored cache values (the reference's tolerance, atol 2e-5 and
     rtol 1e-4); cache rows no row attends hold NaN; a second run gives the same bits; out = q works."""
+    assert _tiles(M, pos0, window)
     q, kc, vc = _inputs(gpu, ct, M, hq, hkv, cap, M * 5 + pos0 + window)
     kg, vg = kc.double().cpu().numpy(), vc.double().cpu().numpy()
     kc[:, pos0 + M:] = float("nan")
@@ -59,17 +91,18 @@ def test_tiles_match_fp64(gpu, ct, M, pos0, window, cap, hq, hkv):
 def test_values_that_are_not_finite_reach_only_the_rows_that_attend_them(gpu, ct, bad):
     """A cached key or value, or a query, that is not finite: every row gets what the same row gets
     from a call of its own (NaN in the same places), so rows before it stay finite."""
-    M, cap, at = 330, 512, 150
+    M, pos0, cap, at = 330, 800, 1152, 150
+    assert _tiles(M, pos0, 0)
     for where in ("k", "v", "q"):
         q, kc, vc = _inputs(gpu, ct, M, 2, 1, cap, 11)
         qd = torch.from_numpy(q).to(gpu)
-        (dict(k=kc, v=vc)[where][0, at] if where != "q" else qd[at])[5] = bad
+        (dict(k=kc, v=vc)[where][0, pos0 + at] if where != "q" else qd[at])[5] = bad
         o1 = torch.full((M, 128), 7.0, device=gpu)
         o2 = torch.full((M, 128), 7.0, device=gpu)
         say(f"attention tiles ct={ct} {bad} in {where}")
-        mt.attention(qd, 128, M, 2, 1, 0, 0, kc, vc, cap, o1, 128, 0.125)
+        mt.attention(qd, 128, M, 2, 1, pos0, 0, kc, vc, cap, o1, 128, 0.125)
         for m in range(128, 192):
-            mt.attention(qd[m:], 128, 1, 2, 1, m, 0, kc, vc, cap, o2[m:], 128, 0.125)
+            mt.attention(qd[m:], 128, 1, 2, 1, pos0 + m, 0, kc, vc, cap, o2[m:], 128, 0.125)
         torch.cuda.synchronize()
         a, b = o1.cpu().numpy()[128:192], o2.cpu().numpy()[128:192]
         assert np.isfinite(a[:at - 128]).all()
@@ -78,16 +111,21 @@ def test_values_that_are_not_finite_reach_only_the_rows_that_attend_them(gpu, ct
 
 def test_large_and_small_queries(gpu):
     """The halves of q are scaled by the row's own power of two: queries of 1e-6 and of 1e5 (past
-    fp16's range), with a score scale that keeps the scores ordinary, and a negative scale."""
-    M, cap = 320, 320
+    fp16's range), with a score scale that keeps the scores ordinary, and a negative scale.  q rows
+    stand in rows of q | k | v, as the engine's do."""
+    M, pos0, cap, ld = 320, 760, 1080, 256
+    assert _tiles(M, pos0, 0)
     for size, scale in ((1e-6, 1.2e5), (1e5, 1.2e-6), (1.0, -0.125)):
         q, kc, vc = _inputs(gpu, torch.float16, M, 2, 1, cap, 3, size)
         out = torch.full((M, 128), 7.0, device=gpu)
+        qkv = torch.full((M, ld), float("nan"), device=gpu)
+        qkv[:, :128] = torch.from_numpy(q).to(gpu)
         say(f"attention tiles q {size} scale {scale}")
-        mt.attention(torch.from_numpy(q).to(gpu), 128, M, 2, 1, 0, 0, kc, vc, cap, out, 128, scale)
+        mt.attention(qkv, ld, M, 2, 1, pos0, 0, kc, vc, cap, out, 128, scale)
         torch.cuda.synchronize()
         for m in (0, 100, M - 1):
-            want = O.attention_f64(q[m].reshape(2, 64), kc.double().cpu().numpy(), vc.double().cpu().numpy(), m, 0, scale)
+            want = O.attention_f64(q[m].reshape(2, 64), kc.double().cpu().numpy(), vc.double().cpu().numpy(), pos0 + m, 0,
+                                   scale)
             ex, i, g, w = O.worst_violation(out[m].cpu().numpy().reshape(2, 64), want, 2e-5)
             assert ex <= 0, f"row {m} index {i} got {g} want {w}"
 
