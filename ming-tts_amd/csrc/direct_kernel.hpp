@@ -20,9 +20,6 @@
 //     x are exact.  One barrier a stage.
 //   - The two halves' sums meet through LDS (first + second), each wave finishing half of the
 //     accumulator registers.
-//   - SPLITK (long K): several workgroups share a tile's K.  Each writes its partial tile in register
-//     order with device-coherent stores and counts itself in; the one that arrives last adds the parts
-//     in order, as tiled_kernel's.
 //   - Bound: the x loads (a lane's 16 bytes are its row's own, so an instruction takes a cycle for each
 //     of its 64 pieces) and, with one tile a CU, a tile's first loads and epilogue.  The same tiles
 //     with x through LDS as fp32 (direct loads) were bound by LDS writes instead and no faster
@@ -55,10 +52,6 @@ struct DirectArgs {
     float eps;
     uint32_t tiles_m, tiles_n;
     uint32_t x_bytes, w_bytes;  // extents of x and of each weight matrix
-    uint32_t splits, kps;       // SPLITK: parts of K, stages of a part
-    float *part;                // their partial tiles
-    uint32_t part_bytes;
-    uint32_t *cnt;              // per-tile arrival counters (zero between launches)
 };
 
 // One wave-wide load to LDS: lane l's 16 bytes at offset voff + soff of the buffer land at LDS byte
@@ -79,28 +72,24 @@ struct Shape {
     static_assert(LPW * NW * 1024 == SB && NS * SB <= 152 * 1024 && XC >= 1, "direct shape");
 };
 
-template <int WT, int WM, int CB, bool GATED, bool NORM, bool SPLITK>
+template <int WT, int WM, int CB, bool GATED, bool NORM>
 __global__ __launch_bounds__(128 * WM, 2) void direct_kernel(DirectArgs a) {
     typedef Shape<WM, CB> S;
     constexpr int FN = GATED ? S::BR / 2 : S::BR;
     static_assert(!GATED || CB % 2 == 0, "gate and up blocks alternate");
-    static_assert(!SPLITK || (!GATED && !NORM), "a split linear is plain");
     __shared__ __attribute__((aligned(1024))) uint8_t lds[NS * S::SB];
     __shared__ __attribute__((aligned(16))) uint16_t gain[NORM ? NORM_K : 8];
     __shared__ float rs[NORM ? 2 * S::BM : 1];
-    __shared__ uint32_t last_flag;
     const int tid = threadIdx.x, lane = tid & 63;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t wm = wave % WM, kh = wave / WM;
     const uint32_t fr = lane & 31, fh = lane >> 5;
 
     const uint32_t t = tiled::xcd_order(blockIdx.x, gridDim.x);
-    const uint32_t tm = t % a.tiles_m, rest = t / a.tiles_m;
-    const uint32_t split = SPLITK ? rest % a.splits : 0, tn = SPLITK ? rest / a.splits : rest;
+    const uint32_t tm = t % a.tiles_m, tn = t / a.tiles_m;
     const uint32_t m0 = tm * S::BM, n0 = tn * FN;
     const uint32_t M = a.M, N = a.N, K = a.K;
-    const uint32_t s0 = SPLITK ? split * a.kps : 0;  // the part's first stage
-    const uint32_t nsteps = SPLITK ? min(a.kps, K / SK - s0) : K / SK;
+    const uint32_t nsteps = K / SK;
 
     const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(a.x), 0, static_cast<int>(a.x_bytes), 0x00020000);
     const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(a.w), 0, static_cast<int>(a.w_bytes), 0x00020000);
@@ -121,7 +110,7 @@ __global__ __launch_bounds__(128 * WM, 2) void direct_kernel(DirectArgs a) {
     const uint32_t lds0 =
         static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) void *)(lds)));
     auto issue = [&](uint32_t s, uint32_t slot) {
-        const uint32_t out = s < nsteps ? 0u : 0x80000000u, so = s < nsteps ? (s0 + s) * (2 * SK) : 0u;
+        const uint32_t out = s < nsteps ? 0u : 0x80000000u, so = s < nsteps ? s * (2 * SK) : 0u;
 #pragma unroll
         for (int i = 0; i < S::LPW; i++) {
             const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0 + slot * S::SB + (wave + S::NW * i) * 1024);
@@ -137,7 +126,7 @@ __global__ __launch_bounds__(128 * WM, 2) void direct_kernel(DirectArgs a) {
     // after: a value that needs all of the registers' old contents (a request that the compiler
     // moves ahead of a last use gets other registers, and the copies back wait for it).
     auto loadx = [&](uint32_t s, u32x4t (&xq)[2], int q, uint32_t after) {
-        const uint32_t so = s < nsteps ? (s0 + s) * (4 * SK) : 0u;
+        const uint32_t so = s < nsteps ? s * (4 * SK) : 0u;
         uint32_t vo = xoff | (s < nsteps ? 0u : 0x80000000u);
         asm volatile("" : "+v"(vo) : "v"(after), "v"(ss[0]), "v"(ss[1]));
         xq[0] = __builtin_bit_cast(u32x4t, __builtin_amdgcn_raw_buffer_load_b128(xr, vo + 64 * q, so, 0));
@@ -283,53 +272,6 @@ __global__ __launch_bounds__(128 * WM, 2) void direct_kernel(DirectArgs a) {
                         sm[j][4 * u + e] = KC == 0 ? own + p[e] : p[e] + own;
                     }
                 }
-        }
-        if constexpr (SPLITK) {
-            // Partial tile: float4 u of block j of wave w at ((w CB + j) 2 + u) 64 + lane.
-            constexpr uint32_t NE = S::BM * S::BR;
-            static_assert(NE == S::NW * CB * 2 * 64 * 4, "partial layout");
-            const __amdgpu_buffer_rsrc_t pr = __builtin_amdgcn_make_buffer_rsrc(a.part, 0, static_cast<int>(a.part_bytes), 0x00020000);
-            const uint32_t tile = tn * a.tiles_m + tm;
-            const uint32_t at0 = (tile * a.splits * NE + (wave * CB * 2 * 64 + lane) * 4) * 4;
-#pragma unroll
-            for (int j = 0; j < CB; j++)
-#pragma unroll
-                for (int u = 0; u < 2; u++)
-                    __builtin_amdgcn_raw_buffer_store_b128(
-                        __builtin_bit_cast(u32x4t, f32x4t{sm[j][4 * u], sm[j][4 * u + 1], sm[j][4 * u + 2], sm[j][4 * u + 3]}), pr,
-                        at0 + split * NE * 4 + (2 * j + u) * 1024, 0, tiled::SC1);
-            tiled::wait_vm<0>();
-            __syncthreads();
-            if (tid == 0) {
-                const uint32_t old = __hip_atomic_fetch_add(a.cnt + tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                last_flag = old == a.splits - 1;
-            }
-            __syncthreads();
-            if (!last_flag) return;
-            if (tid == 0) __hip_atomic_store(a.cnt + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            float tot[CB][RK];
-#pragma unroll
-            for (int j = 0; j < CB; j++)
-#pragma unroll
-                for (int e = 0; e < RK; e++) tot[j][e] = 0.0f;
-            for (uint32_t sp = 0; sp < a.splits; sp++) {
-                f32x4t v[CB][2];
-#pragma unroll
-                for (int j = 0; j < CB; j++)
-#pragma unroll
-                    for (int u = 0; u < 2; u++)
-                        v[j][u] = __builtin_bit_cast(
-                            f32x4t, __builtin_amdgcn_raw_buffer_load_b128(
-                                        pr, sp != split ? at0 + sp * NE * 4 + (2 * j + u) * 1024 : 0xFFFFFFF0u, 0, tiled::SC1));
-#pragma unroll
-                for (int j = 0; j < CB; j++)
-#pragma unroll
-                    for (int e = 0; e < RK; e++) tot[j][e] += sp == split ? sm[j][e] : v[j][e >> 2][e & 3];
-            }
-#pragma unroll
-            for (int j = 0; j < CB; j++)
-#pragma unroll
-                for (int e = 0; e < RK; e++) sm[j][e] = tot[j][e];
         }
         const bool full = m0 + S::BM <= M && n0 + FN <= N;
         const uint32_t flags = a.flags;

@@ -21,13 +21,12 @@ constexpr Tile TILES[] = {{0, 0}, {2, 6}, {4, 6}, {4, 4}};
 template <int WT, bool GATED, bool NORM>
 direct_fn pick(int tile) {
     using direct::direct_kernel;
-    if (tile == 1) return direct_kernel<WT, 2, 6, GATED, NORM, false>;
-    if (GATED || tile == 2) return direct_kernel<WT, 4, 6, GATED, NORM, false>;
-    return direct_kernel<WT, 4, 4, false, NORM, false>;
+    if (tile == 1) return direct_kernel<WT, 2, 6, GATED, NORM>;
+    if (GATED || tile == 2) return direct_kernel<WT, 4, 6, GATED, NORM>;
+    return direct_kernel<WT, 4, 4, false, NORM>;
 }
 template <int WT>
-direct_fn pick_wt(bool gated, bool norm, int tile, uint32_t splits) {
-    if (splits > 1) return direct::direct_kernel<WT, 2, 6, false, false, true>;  // tile 1
+direct_fn pick_wt(bool gated, bool norm, int tile) {
     if (gated) return norm ? pick<WT, true, true>(tile) : pick<WT, true, false>(tile);
     return norm ? pick<WT, false, true>(tile) : pick<WT, false, false>(tile);
 }
@@ -52,23 +51,12 @@ bool direct_takes(const LinearArgs &a) {
 // 192 rows), on the 128-row tiles where ring_fills (linear_gemm_lds.hip) says that they fill the
 // chip; others once tiled_kernel's 64 x 128 tiles no longer do, and the tile with the least estimate
 // takes it.  64 x 128 tiles of this kernel were ahead of tiled_kernel's in a graph of their own (qkv at
-// 1600 rows 15.7 against 16.5 us) but not where x comes from the kernel before (19.7 against 17.4).
-// Long K (2048 and more, no gate and no norm) from 1024 rows: 64 x 192 tiles with K in as many parts as
-// keep the workgroups in one wave, at least two (down at 1024 rows in 3 parts 31.8 against 36.3 us in
-// tiled_kernel's, at 1600 in 2 47.6 against 54.4; the audio encoder's layer 187.8 -> 182.2 us).  Not at
-// two workgroups a CU: down at 2048 rows in 3 parts was ahead in a graph of its own (56.7 against 66.4
-// us) and behind after the kernels before it (one layer 237 -> 248 us).  At 512 rows 24.5 against 23.4.
-int direct_tile(const LinearArgs &a, int cus, bool ring_fills, uint32_t &splits) {
-    splits = 1;
-    if (!direct_takes(a) || a.K < 512) return 0;
+// 1600 rows 15.7 against 16.5 us) but not where x comes from the kernel before (19.7 against 17.4), and
+// with long K they were behind (down at 2048 rows 70 against 63 us): tiled_kernel keeps x further ahead.
+int direct_tile(const LinearArgs &a, int cus, bool ring_fills) {
+    if (!direct_takes(a) || a.K < 512 || a.K >= 2048) return 0;
     const bool gated = (a.flags & F_SILU_GATE) != 0;
     const uint32_t ncu = static_cast<uint32_t>(cus);
-    if (a.K >= 2048) {
-        const uint64_t tiles = static_cast<uint64_t>((a.M + 63) / 64) * ((a.N + 191) / 192);
-        if (gated || a.norm || a.M < 1024 || 2 * tiles > ncu) return 0;
-        splits = std::min(ncu / static_cast<uint32_t>(tiles), a.K / (8 * direct::SK));  // parts of at least 8 stages
-        return 1;
-    }
     const auto waves = [&](uint32_t bm, uint32_t fn) {
         return (((a.M + bm - 1) / bm) * ((a.N + fn - 1) / fn) + ncu - 1) / ncu;
     };
@@ -83,12 +71,7 @@ int direct_tile(const LinearArgs &a, int cus, bool ring_fills, uint32_t &splits)
     return c1 <= c2 && c1 <= c3 ? 1 : c2 <= c3 ? 2 : 3;
 }
 
-size_t direct_partial_bytes(const LinearArgs &a, int tile, uint32_t splits) {
-    const uint64_t bm = 32 * TILES[tile].wm, br = 32 * TILES[tile].cb;
-    return ((a.M + bm - 1) / bm) * ((a.N + br - 1) / br) * splits * bm * br * sizeof(float);
-}
-
-int launch_gemm_direct(const LinearArgs &a, int wt, int tile, uint32_t splits, hipStream_t stream, const FixedWs *fixed) {
+int launch_gemm_direct(const LinearArgs &a, int wt, int tile, hipStream_t stream) {
     const bool gated = (a.flags & F_SILU_GATE) != 0;
     const uint32_t bm = 32 * TILES[tile].wm, fn = (gated ? 16 : 32) * TILES[tile].cb;
     DirectArgs t;
@@ -104,23 +87,9 @@ int launch_gemm_direct(const LinearArgs &a, int wt, int tile, uint32_t splits, h
     t.tiles_n = (a.N + fn - 1) / fn;
     t.x_bytes = static_cast<uint32_t>((static_cast<uint64_t>(a.M - 1) * a.ldx + a.K) * 4);
     t.w_bytes = a.N * a.K * 2;
-    const uint32_t stages = a.K / direct::SK;
-    t.kps = (stages + splits - 1) / splits;
-    t.splits = (stages + t.kps - 1) / t.kps;
-    t.part = nullptr;
-    t.part_bytes = 0;
-    t.cnt = nullptr;
-    if (t.splits > 1) {
-        void *part = nullptr;
-        const size_t pb = direct_partial_bytes(a, tile, t.splits);
-        const int rc = split_workspace(fixed, stream, pb, t.tiles_m * t.tiles_n, &part, &t.cnt, "gemm");
-        if (rc) return rc;
-        t.part = static_cast<float *>(part);
-        t.part_bytes = static_cast<uint32_t>(pb);
-    }
-    const uint64_t G = static_cast<uint64_t>(t.tiles_m) * t.tiles_n * t.splits;
+    const uint64_t G = static_cast<uint64_t>(t.tiles_m) * t.tiles_n;
     if (G == 0 || G > 0x7FFFFFFFu) return set_error(MT_EINVAL, "gemm: %llu direct tiles", static_cast<unsigned long long>(G));
-    direct_fn kernel = wt == DT_BF16 ? pick_wt<DT_BF16>(gated, a.norm != nullptr, tile, t.splits) : pick_wt<DT_F16>(gated, a.norm != nullptr, tile, t.splits);
+    direct_fn kernel = wt == DT_BF16 ? pick_wt<DT_BF16>(gated, a.norm != nullptr, tile) : pick_wt<DT_F16>(gated, a.norm != nullptr, tile);
     hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(G)), dim3(128 * TILES[tile].wm), 0, stream, t);
     return check_launch("gemm (direct)");
 }

@@ -140,15 +140,11 @@ int launch_gemm_tiled(const LinearArgs &a, int xt, int wt, hipStream_t stream, c
     if (cus <= 0) return set_error(MT_EHIP, "gemm: cannot query the device");
     const int tile = tuning().gemm_tile, splitk = tuning().gemm_splitk, stages_override = tuning().gemm_stages;
     if (split && tile == 0 && splitk == 0 && stages_override == 0) {
-        uint32_t parts = 1;
-        const int d = direct_tile(a, cus, gated && ring_fills(a.M, a.N, cus), parts);
-        // Parts of K need a workspace that tiled_plan's kernel may not: where there is none to be had
-        // (a smaller static scratch, growth under graph capture) the linear stays there.
-        if (d && (parts == 1 || workspace_ready(fixed, stream, direct_partial_bytes(a, d, parts))))
-            return launch_gemm_direct(a, wt, d, parts, stream, fixed);
+        const int d = direct_tile(a, cus, gated && ring_fills(a.M, a.N, cus));
+        if (d) return launch_gemm_direct(a, wt, d, stream);
     }
     // The gated 128 x 96 tiles by request: fp32 x on the direct kernel where it takes the linear.
-    if (split && gated && tile == 5 && direct_takes(a)) return launch_gemm_direct(a, wt, 2, 1, stream, fixed);
+    if (split && gated && tile == 5 && direct_takes(a)) return launch_gemm_direct(a, wt, 2, stream);
     if (gated && !split && (tile == 5 || (tile == 0 && splitk == 0 && ring_fills(a.M, a.N, cus)))) {
         ring::RingArgs r{};
         r.x = static_cast<const uint16_t *>(a.x);

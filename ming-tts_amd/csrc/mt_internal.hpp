@@ -176,9 +176,6 @@ int static_scratch(hipStream_t stream, FixedWs &ws);
 // The split-K workspace of a launch: the fixed scratch when fixed != null, else the stream's.
 int split_workspace(const FixedWs *fixed, hipStream_t stream, size_t part_bytes, uint32_t counters, void **part,
                     uint32_t **cnt, const char *who);
-// Would split_workspace give part_bytes (and up to 1024 counters) now: it fits the fixed scratch, or the
-// stream's workspace, or that may grow (at most 2 GiB, and not while the stream is being captured)?
-bool workspace_ready(const FixedWs *fixed, hipStream_t stream, size_t part_bytes);
 
 // Compute units of the current device (cached per device), or <= 0 when it cannot be queried.
 int device_cus();
@@ -200,11 +197,9 @@ TiledPlan tiled_plan(uint32_t M, uint32_t N, uint32_t K, bool gated, int cus, in
 int launch_gemm_tiled(const LinearArgs &a, int xt, int wt, hipStream_t stream, const FixedWs *fixed = nullptr);
 
 // The direct GEMM for fp32 x over many rows (direct_kernel.hpp): whether it can take a linear, the tile
-// it takes one in (0: it is left to tiled_plan's kernels) with the parts of K, the bytes of their
-// partial tiles, and its launch.
+// it takes one in (0: it is left to tiled_plan's kernels), and its launch.
 bool direct_takes(const LinearArgs &a);
-int direct_tile(const LinearArgs &a, int cus, bool ring_fills, uint32_t &splits);
-size_t direct_partial_bytes(const LinearArgs &a, int tile, uint32_t splits);
-int launch_gemm_direct(const LinearArgs &a, int wt, int tile, uint32_t splits, hipStream_t stream, const FixedWs *fixed);
+int direct_tile(const LinearArgs &a, int cus, bool ring_fills);
+int launch_gemm_direct(const LinearArgs &a, int wt, int tile, hipStream_t stream);
 
 }  // namespace mt

@@ -58,25 +58,6 @@ int split_workspace(const FixedWs *fixed, hipStream_t stream, size_t part_bytes,
     return MT_OK;
 }
 
-bool workspace_ready(const FixedWs *fixed, hipStream_t stream, size_t part_bytes) {
-    constexpr uint32_t counters = 1024;  // what the first allocation holds at least
-    if (fixed) return part_bytes <= fixed->part_bytes && counters <= fixed->counters;
-    if (part_bytes > 0x7FFFFFF0u) return false;
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return false;
-    {
-        std::lock_guard<std::mutex> lock(g_ws_mu);
-        const auto it = g_ws.find(std::make_pair(dev, stream));
-        if (it != g_ws.end() && it->second.base && it->second.part_bytes >= part_bytes) return true;
-    }
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(stream, &cs) != hipSuccess) {  // e.g. the legacy stream beside a global capture
-        (void)hipGetLastError();  // not the launch's error
-        return false;
-    }
-    return cs == hipStreamCaptureStatusNone;
-}
-
 int stream_workspace(hipStream_t stream, size_t part_bytes, uint32_t counters, void **part, uint32_t **cnt) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return set_error(MT_EHIP, "workspace: no current device");
