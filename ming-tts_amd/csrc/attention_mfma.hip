@@ -76,6 +76,22 @@ struct AmType {
     static constexpr float PS = CT == DT_F16 ? 16384.0f : 1.0f;  // the weights' scale
 };
 
+// Eight values of q or p as the operand's pieces.
+template <int CT>
+__device__ __forceinline__ void pieces(const float (&x)[8], u32x4t (&p)[AmType<CT>::NQ]) {
+    if constexpr (CT == DT_F16) {
+        tiled::split8<DT_F16, true>(x, p[0], p[1]);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            uint32_t w[3];
+            split3(x[2 * e], x[2 * e + 1], w);
+#pragma unroll
+            for (int i = 0; i < 3; i++) p[i][e] = w[i];
+        }
+    }
+}
+
 // The products of a sum: every piece of q (or p) against an fp16 k (or v); of three pieces against
 // three, the six that are not below 2^-24.  am_small adds all but the largest (all below 2^-8 of
 // it); a sum takes those of every step first and then the largest, so it rounds at its own size
@@ -145,21 +161,8 @@ __global__ __launch_bounds__(AM_THREADS, 2) void attention_mfma_kernel(
 #pragma unroll
     for (int kk = 0; kk < 4; kk++) {
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const float x0 = x[kk][2 * e] * f, x1 = x[kk][2 * e + 1] * f;
-            if constexpr (CT == DT_F16) {
-                uint32_t hw, lw;
-                tiled::split2<DT_F16>(x0, x1, hw, lw);
-                qf[kk][0][e] = hw;
-                qf[kk][1][e] = lw;
-            } else {
-                uint32_t p[3];
-                split3(x0, x1, p);
-#pragma unroll
-                for (int i = 0; i < 3; i++) qf[kk][i][e] = p[i];
-            }
-        }
-        tiled::settle<TY::MT>(qf[kk][1]);
+        for (int e = 0; e < 8; e++) x[kk][e] *= f;
+        pieces<CT>(x[kk], qf[kk]);
     }
 
     f32x16t o[2];
@@ -264,24 +267,12 @@ __global__ __launch_bounds__(AM_THREADS, 2) void attention_mfma_kernel(
         ls = fmaf(ls, al, sum);
         u32x4t pf[2][TY::NQ];
 #pragma unroll
-        for (int kk = 0; kk < 2; kk++)
+        for (int kk = 0; kk < 2; kk++) {
+            float x8[8];
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const float x0 = p[8 * kk + 2 * e] * TY::PS, x1 = p[8 * kk + 2 * e + 1] * TY::PS;
-                if constexpr (CT == DT_F16) {
-                    uint32_t hw, lw;
-                    tiled::split2<DT_F16>(x0, x1, hw, lw);
-                    pf[kk][0][e] = hw;
-                    pf[kk][1][e] = lw;
-                } else {
-                    uint32_t w[3];
-                    split3(x0, x1, w);
-#pragma unroll
-                    for (int i = 0; i < 3; i++) pf[kk][i][e] = w[i];
-                }
-            }
-        tiled::settle<TY::MT>(pf[0][1]);
-        tiled::settle<TY::MT>(pf[1][1]);
+            for (int e = 0; e < 8; e++) x8[e] = p[8 * kk + e] * TY::PS;
+            pieces<CT>(x8, pf[kk]);
+        }
 
         // p . v: d = 0 the even dims, 1 the odd ones.  A tile's sum starts from zero and joins the
         // running one in one rounding.

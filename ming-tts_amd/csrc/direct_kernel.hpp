@@ -203,8 +203,7 @@ __global__ __launch_bounds__(128 * WM, 2) void direct_kernel(DirectArgs a) {
                 }
             }
             u32x4t ah, al;
-            tiled::split8<WT>(x, ah, al);
-            tiled::settle<WT>(al);
+            tiled::split8<WT, true>(x, ah, al);
             loadx(s + 2, xs[q], q, al[3]);
 #pragma unroll
             for (int j = 0; j < CB; j++) acc[j] = tiled::mfma32x<WT>(al, b[j], acc[j]);

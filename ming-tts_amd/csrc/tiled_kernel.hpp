@@ -125,42 +125,55 @@ __device__ __forceinline__ uint32_t xcd_order(uint32_t b, uint32_t G) {
 // (fp32 x minus the fp16 hi, rounded to fp16 into the pair's low or high half) after one
 // packed conversion for the pair's hi: 3 instructions a pair.  bf16 has no mixed fma: the
 // pair's hi is widened back and subtracted.
+//
+// MFMA: lo goes to an MFMA as it is rather than to LDS.  An MFMA needs two wait states after a vector
+// instruction that wrote an operand.  The compiler keeps them for its own instructions, but behind
+// inline asm it keeps one only (what any vector instruction needs after a write to half a register),
+// so the eight fmas are then one block that ends with two; lo takes the registers of the even x.  Where
+// lo goes to LDS the single fmas are left to the scheduler: as a block they cost the tiled kernel 2-3 %
+// (down at 174 rows 14.65 -> 15.03 us, o at 1600 15.2 -> 15.65).
 typedef float f32x2t __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x2t __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2t __attribute__((ext_vector_type(2)));
-template <int T>
-__device__ __forceinline__ void split2(float x0, float x1, uint32_t &hi, uint32_t &lo) {
-    if constexpr (T == DT_BF16) {
-        const uint32_t h = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2t{x0, x1}, bf16x2t));
-        hi = h;
-        lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2t{x0 - bf16_lo(h), x1 - bf16_hi(h)}, bf16x2t));
-    } else {
-        const uint32_t h = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2t{x0, x1}, f16x2t));
-        uint32_t l;
-        asm("v_fma_mixlo_f16 %0, %1, 1.0, -%2 op_sel_hi:[0,0,1]" : "=v"(l) : "v"(x0), "v"(h));
-        asm("v_fma_mixhi_f16 %0, %1, 1.0, -%2 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "+v"(l) : "v"(x1), "v"(h));
-        hi = h;
-        lo = l;
-    }
-}
-template <int T>
+template <int T, bool MFMA = false>
 __device__ __forceinline__ void split8(const float (&x)[8], u32x4t &hi, u32x4t &lo) {
+    uint32_t h[4], l[4];
+    if constexpr (T == DT_BF16) {
 #pragma unroll
-    for (int e = 0; e < 4; e++) {
-        uint32_t h, l;
-        split2<T>(x[2 * e], x[2 * e + 1], h, l);
-        hi[e] = h;
-        lo[e] = l;
+        for (int e = 0; e < 4; e++) {
+            h[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2t{x[2 * e], x[2 * e + 1]}, bf16x2t));
+            l[e] = __builtin_bit_cast(
+                uint32_t, __builtin_convertvector(f32x2t{x[2 * e] - bf16_lo(h[e]), x[2 * e + 1] - bf16_hi(h[e])}, bf16x2t));
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            h[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2t{x[2 * e], x[2 * e + 1]}, f16x2t));
+        if constexpr (MFMA) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) l[e] = __float_as_uint(x[2 * e]);
+            asm("v_fma_mixlo_f16 %0, %0, 1.0, -%4 op_sel_hi:[0,0,1]\n\t"
+                "v_fma_mixlo_f16 %1, %1, 1.0, -%5 op_sel_hi:[0,0,1]\n\t"
+                "v_fma_mixlo_f16 %2, %2, 1.0, -%6 op_sel_hi:[0,0,1]\n\t"
+                "v_fma_mixlo_f16 %3, %3, 1.0, -%7 op_sel_hi:[0,0,1]\n\t"
+                "v_fma_mixhi_f16 %0, %8, 1.0, -%4 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+                "v_fma_mixhi_f16 %1, %9, 1.0, -%5 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+                "v_fma_mixhi_f16 %2, %10, 1.0, -%6 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+                "v_fma_mixhi_f16 %3, %11, 1.0, -%7 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+                "s_nop 1"
+                : "+&v"(l[0]), "+&v"(l[1]), "+&v"(l[2]), "+&v"(l[3])
+                : "v"(h[0]), "v"(h[1]), "v"(h[2]), "v"(h[3]), "v"(x[1]), "v"(x[3]), "v"(x[5]), "v"(x[7]));
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                asm("v_fma_mixlo_f16 %0, %1, 1.0, -%2 op_sel_hi:[0,0,1]" : "=v"(l[e]) : "v"(x[2 * e]), "v"(h[e]));
+                asm("v_fma_mixhi_f16 %0, %1, 1.0, -%2 op_sel:[0,0,1] op_sel_hi:[0,0,1]"
+                    : "+v"(l[e]) : "v"(x[2 * e + 1]), "v"(h[e]));
+            }
+        }
     }
-}
-
-// Between split8 and a VALU or MFMA instruction that reads lo: v_fma_mixhi moves its result to the
-// upper half of the register, and such a result takes one wait state before the next vector
-// instruction may read it.  The compiler inserts it for its own instructions, but does not look
-// into inline asm.  (Stores to LDS need none.)
-template <int T>
-__device__ __forceinline__ void settle(u32x4t &lo) {
-    if constexpr (T == DT_F16) asm("s_nop 0" : "+v"(lo));
+    hi = u32x4t{h[0], h[1], h[2], h[3]};
+    lo = u32x4t{l[0], l[1], l[2], l[3]};
 }
 
 template <int BM, int BN, bool GATED, int KS, bool SPLIT>
