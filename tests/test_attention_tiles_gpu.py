@@ -109,6 +109,29 @@ def test_values_that_are_not_finite_reach_only_the_rows_that_attend_them(gpu, ct
         np.testing.assert_allclose(a, b, rtol=1e-4, atol=2e-5)
 
 
+@pytest.mark.parametrize("M,pos0,window", [(700, 1024, 0), (400, 0, 65)])
+@pytest.mark.parametrize("ct", [torch.float16, torch.float32])
+def test_values_with_a_mean_are_as_exact_as_by_the_row_kernel(gpu, ct, M, pos0, window):
+    """Values of one sign: sums that round towards zero above the fraction and to nearest below it would
+    show.  The error against fp64 stays within that of the same rows in calls of their own (a tenth more
+    for the sample's size: 0.8 to 1.0 of it measured)."""
+    assert _tiles(M, pos0, window)
+    cap = pos0 + M
+    q, kc, vc = _inputs(gpu, ct, M, 2, 1, cap, 13, 3.0)
+    vc += 5.0
+    qd = torch.from_numpy(q).to(gpu)
+    o1, o2 = torch.full((M, 128), 7.0, device=gpu), torch.full((M, 128), 7.0, device=gpu)
+    say(f"attention tiles ct={ct} values with a mean M={M} pos0={pos0} window={window}")
+    mt.attention(qd, 128, M, 2, 1, pos0, window, kc, vc, cap, o1, 128, 0.125)
+    for m in range(M):
+        mt.attention(qd[m:], 128, 1, 2, 1, pos0 + m, window, kc, vc, cap, o2[m:], 128, 0.125)
+    torch.cuda.synchronize()
+    kg, vg = kc.double().cpu().numpy(), vc.double().cpu().numpy()
+    want = np.stack([O.attention_f64(q[m].reshape(2, 64), kg, vg, pos0 + m, window, 0.125).reshape(128) for m in range(M)])
+    e1, e2 = (np.linalg.norm(o.double().cpu().numpy() - want) for o in (o1, o2))
+    assert e1 <= 1.1 * e2, f"{e1 / e2:.2f}"
+
+
 def test_large_and_small_queries(gpu):
     """The halves of q are scaled by the row's own power of two: queries of 1e-6 and of 1e5 (past
     fp16's range), with a score scale that keeps the scores ordinary, and a negative scale.  q rows
