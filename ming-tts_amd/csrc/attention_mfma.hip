@@ -25,17 +25,17 @@
 //     at 400 to 2048 rows, windows of 5 and 65 and none, queries of 0.1 to 40; values with a mean
 //     0.89-1.01 / 0.82-0.87 (1.3 / 1.05 with the weights summed beside the MFMAs, which takes 0.1-1 us
 //     less, 4 less at 4000 fp16 keys, and 1.1 more at 1600 fp16 rows of window 65).
-//   - Results do not depend on how rows fall into blocks: tiles start at multiples of 32 keys,
-//     a tile without keys of a row adds exact zeros to it, and the four waves' parts meet in
-//     wave order.
+//   - Tiles start at multiples of 32 keys, a tile without keys of a row adds exact zeros to it, and
+//     the four waves' parts meet in wave order: a row's result does not depend on the block it falls
+//     into while the cache rows that the block reads are finite.
 //   - Bound: a wave's own instructions (about 240 a tile beside 16 MFMAs with an fp16 cache) and,
 //     with few tiles a wave, its loads' latency.  2048 rows from position 0 (14 / 2 heads, graph
 //     replay): 31 us with an fp16 cache, 64 us with an fp32 one (row kernels 431 and 766).  Two row
 //     tiles a wave, which halve the key and value reads, took 256 registers and 36-59 us; three
 //     waves a SIMD spill (38 us).
-//   - An output that is not finite (infinities and NaN in the inputs, or in cache rows that the
-//     row does not attend but its block reads) makes the workgroup redo its rows with the row
-//     kernel's arithmetic, which touches only each row's own keys.
+//   - A row with an output that is not finite (infinities and NaN in its query or keys, or in cache
+//     rows that it does not attend but its block reads) is done again with the row kernel's arithmetic,
+//     which touches only the row's own keys.
 #include "attend_row.hpp"
 #include "mt_device.hpp"
 #include "mt_internal.hpp"
@@ -121,8 +121,7 @@ __global__ __launch_bounds__(AM_THREADS, 2) void attention_mfma_kernel(
     constexpr int ES = CT == DT_F16 ? 2 : 4;  // bytes of a cached value
     __shared__ __attribute__((aligned(16))) float part[AM_WAVES * 32 * AM_OLD];
     __shared__ float mls[2][AM_WAVES][32];
-    __shared__ uint32_t redo;
-    __shared__ uint32_t bad;
+    __shared__ uint32_t redo;  // the block's rows (bits) whose outputs are not finite
     static_assert(sizeof(part) >= sizeof(RowLds), "the row kernel's scratch overlays the hand-over");
     const int tid = threadIdx.x, lane = tid & 63;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -131,7 +130,6 @@ __global__ __launch_bounds__(AM_THREADS, 2) void attention_mfma_kernel(
     const uint32_t m0 = (gridDim.y - 1 - blockIdx.y) * AM_ROWS;  // the longest rows first
     const uint32_t rn = min(AM_ROWS, rows - m0);
     const uint32_t kend = pos0 + m0 + rn;  // keys the block attends end here
-    if (tid == 0) bad = 0;
 
     // The query rows (rows past the end repeat the last one and are never stored), their keys
     // [lo, lo + span) and the factor that turns a dot into a base-2 exponent.
@@ -358,24 +356,23 @@ __global__ __launch_bounds__(AM_THREADS, 2) void attention_mfma_kernel(
         acc[e] *= il;
         ok = ok && fabsf(acc[e]) < INFINITY;
     }
-    // Nothing is stored before the whole workgroup knows that its rows are finite: out may be q.
-    if (mine && !ok) redo = 1;
+    if (mine && !ok) atomicOr(&redo, 1u << row);
     __syncthreads();
-    if (redo) {
-        RowLds *rl = reinterpret_cast<RowLds *>(part);
-        for (uint32_t r = 0; r < rn; r++) {
-            const uint32_t end = pos0 + m0 + r + 1, first = window > 0 && end > window ? end - window : 0;
-            attend_row<CT, 2, 2>(q + static_cast<size_t>(m0 + r) * ldq + h * 64, kc, vc,
-                                 (static_cast<size_t>(kvh) * cache_len + first) * 64, static_cast<int>(end - first), scale,
-                                 out + static_cast<size_t>(m0 + r) * ldo + h * 64, rl->sc, rl->red, rl->part);
-            __syncthreads();
-        }
-        return;
-    }
-    if (mine) {
+    const uint32_t again = redo;
+    if (mine && !((again >> row) & 1)) {
         float *orow = out + static_cast<size_t>(m0 + row) * ldo + h * 64 + 8 * d8;
         *reinterpret_cast<float4 *>(orow) = make_float4(acc[0], acc[1], acc[2], acc[3]);
         *reinterpret_cast<float4 *>(orow + 4) = make_float4(acc[4], acc[5], acc[6], acc[7]);
+    }
+    // The rest once more, a row's query still in place also where out is q.
+    for (uint32_t left = again; left; left &= left - 1) {
+        RowLds *rl = reinterpret_cast<RowLds *>(part);
+        const uint32_t r = __builtin_ctz(left);
+        const uint32_t end = pos0 + m0 + r + 1, first = window > 0 && end > window ? end - window : 0;
+        attend_row<CT, 2, 2>(q + static_cast<size_t>(m0 + r) * ldq + h * 64, kc, vc,
+                             (static_cast<size_t>(kvh) * cache_len + first) * 64, static_cast<int>(end - first), scale,
+                             out + static_cast<size_t>(m0 + r) * ldo + h * 64, rl->sc, rl->red, rl->part);
+        __syncthreads();
     }
 }
 

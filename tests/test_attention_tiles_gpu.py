@@ -109,6 +109,30 @@ def test_values_that_are_not_finite_reach_only_the_rows_that_attend_them(gpu, ct
         np.testing.assert_allclose(a, b, rtol=1e-4, atol=2e-5)
 
 
+@pytest.mark.parametrize("ct", [torch.float16, torch.float32])
+def test_rows_beside_one_that_is_not_finite_keep_their_bits(gpu, ct):
+    """Queries with a NaN and an infinity in rows of their own: every other row of their blocks has the
+    bits of a call without them, also where out is q."""
+    M, pos0, cap = 330, 800, 1152
+    assert _tiles(M, pos0, 0)
+    q, kc, vc = _inputs(gpu, ct, M, 2, 1, cap, 12)
+    qd = torch.from_numpy(q).to(gpu)
+    want = torch.full((M, 128), 7.0, device=gpu)
+    say(f"attention tiles ct={ct} rows beside NaN")
+    mt.attention(qd, 128, M, 2, 1, pos0, 0, kc, vc, cap, want, 128, 0.125)
+    qd[150, 5], qd[159, 70], qd[329, 0] = float("nan"), float("inf"), float("nan")
+    out = torch.full((M, 128), 7.0, device=gpu)
+    mt.attention(qd, 128, M, 2, 1, pos0, 0, kc, vc, cap, out, 128, 0.125)
+    mt.attention(qd, 128, M, 2, 1, pos0, 0, kc, vc, cap, qd, 128, 0.125)
+    torch.cuda.synchronize()
+    bad = np.zeros((M, 2), bool)  # (row, head)
+    bad[150, 0] = bad[159, 1] = bad[329, 0] = True
+    for got in (out, qd):
+        a, b = got.cpu().numpy().reshape(M, 2, 64), want.cpu().numpy().reshape(M, 2, 64)
+        np.testing.assert_array_equal(a[~bad], b[~bad])
+        assert np.isnan(a[bad]).all()
+
+
 @pytest.mark.parametrize("M,pos0,window", [(700, 1024, 0), (400, 0, 65)])
 @pytest.mark.parametrize("ct", [torch.float16, torch.float32])
 def test_values_with_a_mean_are_as_exact_as_by_the_row_kernel(gpu, ct, M, pos0, window):
