@@ -71,20 +71,21 @@ int stream_workspace(hipStream_t stream, size_t part_bytes, uint32_t counters, v
         const size_t pb = std::max(part_bytes, w.part_bytes * 2);
         const uint32_t nc = std::max<uint32_t>(std::max(counters, w.counters * 2), 1024);
         const size_t cb = (static_cast<size_t>(nc) * 4 + COUNTER_BYTES_ALIGN - 1) / COUNTER_BYTES_ALIGN * COUNTER_BYTES_ALIGN;
-        if (w.base) {
-            g_retired.push_back(w.base);  // graphs captured on this stream may still use it
-            w.base = nullptr;
-        }
         void *p = nullptr;
         hipError_t e = hipMalloc(&p, cb + pb);
-        if (e != hipSuccess) return set_error(MT_ENOMEM, "workspace: hipMalloc(%zu): %s", cb + pb, hipGetErrorString(e));
+        if (e != hipSuccess) {
+            (void)hipGetLastError();  // reported here, not by the next launch
+            return set_error(MT_ENOMEM, "workspace: hipMalloc(%zu): %s", cb + pb, hipGetErrorString(e));
+        }
         // Ordered on the stream itself (which need not synchronise with the null stream).
         e = hipMemsetAsync(p, 0, cb, stream);
         if (e == hipSuccess) e = hipStreamSynchronize(stream);
         if (e != hipSuccess) {
             (void)hipFree(p);
+            (void)hipGetLastError();
             return set_error(MT_EHIP, "workspace: hipMemset: %s", hipGetErrorString(e));
         }
+        if (w.base) g_retired.push_back(w.base);  // graphs captured on this stream may still use it
         w.base = p;
         w.part_bytes = pb;
         w.counters = static_cast<uint32_t>(cb / 4);
