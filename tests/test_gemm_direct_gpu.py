@@ -10,20 +10,43 @@ from _gpu_util import say
 
 pytestmark = pytest.mark.gpu
 
-# M, N, K, gated, norm: 64 x 96 features (gated), 128 x 96 (gated, and one past its last wave), 64 x
-# 192, 128 x 192 and 128 x 128 weight rows, with ragged rows and features; odd and even stage counts
-# (8, 14, 15, 31); the shortest and the longest K.
-CASES = [(257, 4864, 896, True, True), (330, 4800, 512, True, False), (513, 4850, 896, True, True), (1793, 1152, 896, False, True),
-         (1601, 3072, 1024, False, True), (900, 4096, 1024, False, True), (1100, 4099, 512, False, False),
-         (2047, 1031, 1984, False, False), (1300, 4099, 960, False, True)]
+# M, N, K, gated, norm and the tile on 256 CUs (1: 64 x 96 features or 64 x 192 weight rows, 2: 128 x 96
+# or 128 x 192, 3: 128 x 128), with ragged rows and features, one gated past its last wave; odd and even
+# stage counts (8, 14, 15, 16, 31); the shortest and the longest K.
+CASES = [(257, 4864, 896, True, True, 1), (330, 4800, 512, True, False, 2), (513, 4850, 896, True, True, 2),
+         (1025, 4864, 896, True, True, 2), (1793, 1152, 896, False, True, 1), (1601, 3072, 1024, False, True, 2),
+         (900, 4096, 1024, False, True, 3), (1100, 4099, 512, False, False, 2), (2047, 1031, 1984, False, False, 1),
+         (1300, 4099, 960, False, True, 2)]
+
+
+def _tile(M, N, K, gated, norm, cus):
+    """linear_gemm_direct.hip's choice: the kernel's tile, 0 for the tiled kernel's linears."""
+    if K % 64 or K < 512 or K >= 2048:
+        return 0
+    tiles = lambda bm, fn: -(-M // bm) * -(-N // fn)  # noqa: E731
+    waves = lambda bm, fn: -(-tiles(bm, fn) // cus)  # noqa: E731
+    if gated:
+        if waves(64, 64) <= 1:
+            return 0
+        if 4 * tiles(128, 96) >= 3 * waves(128, 96) * cus:
+            return 2
+        r1 = waves(64, 96)
+        return 1 if (175 if r1 == 1 else 290 + 150 * (r1 - 2)) <= 260 * waves(128, 96) else 2
+    if waves(64, 128) <= 1:
+        return 0
+    cost = [20 + 170 * waves(64, 192), 30 + 260 * waves(128, 192), 245 * waves(128, 128)]
+    return 1 + cost.index(min(cost))
 
 
 @pytest.mark.parametrize("wt", [O.F16, O.BF16], ids=["wf16", "wbf16"])
-@pytest.mark.parametrize("M,N,K,gated,norm", CASES)
-def test_direct_gemm_matches_fp64(gpu, M, N, K, gated, norm, wt):
+@pytest.mark.parametrize("M,N,K,gated,norm,tile", CASES)
+def test_direct_gemm_matches_fp64(gpu, M, N, K, gated, norm, tile, wt):
     """x in a wider matrix (ldx > K) with NaN between its rows, y in a wider one that keeps what lies
     between, bias and accumulate; normwise within the bound of x in two halves (2^-22 of x with fp16,
-    2^-17 with bf16) plus fp32 sums, and twice the same bits."""
+    2^-17 with bf16) plus fp32 sums, and twice the same bits.  The bits are those of no tile of the tiled
+    kernel, which sums in another order, and mt_linear_static gives them too."""
+    cus = torch.cuda.get_device_properties(gpu).multi_processor_count
+    assert _tile(M, N, K, gated, norm, cus) == tile or cus != 256
     say(f"direct gemm {M}x{N}x{K} gated={gated} norm={norm} w{wt}")
     dt = torch.float16 if wt == O.F16 else torch.bfloat16
     g = torch.Generator(device=gpu)
@@ -36,14 +59,29 @@ def test_direct_gemm_matches_fp64(gpu, M, N, K, gated, norm, wt):
     b, gain = rand(N, sc=0.1).to(dt), (1.0 + 0.1 * rand(K)).to(dt)
     y0 = rand(M, ldy)
     flags = mt.GemvFlags.accumulate | (mt.GemvFlags.siluGate if gated else 0)
-    runs = []
-    for _ in range(2):
+
+    def run(tile=0):
         y = y0.clone()
-        mt.linear(xs, w, y, flags=flags, w2=w2 if gated else None, bias=b, ldx=ldx, ldy=ldy, norm=gain if norm else None)
+        old = mt.set_tuning(mt.TUNE_GEMM_TILE, tile)
+        try:
+            mt.linear(xs, w, y, flags=flags, w2=w2 if gated else None, bias=b, ldx=ldx, ldy=ldy, norm=gain if norm else None)
+        finally:
+            mt.set_tuning(mt.TUNE_GEMM_TILE, old)
         torch.cuda.synchronize()
-        runs.append(y)
+        return y
+
+    runs = [run(), run()]
     assert torch.equal(runs[0], runs[1])
     assert torch.equal(runs[0][:, N:], y0[:, N:])
+    for tiled in (1, 2) if gated else (1, 2, 3):
+        assert not torch.equal(runs[0], run(tiled)), tiled
+    if not norm:
+        y = y0.clone()
+        rc = mt.linear_static_raw(xs, mt.F32, w, w2 if gated else None, mt.F16 if wt == O.F16 else mt.BF16, b, y, M, N, K, ldx,
+                                  ldy, flags)
+        assert rc == mt.OK, mt.last_error()
+        torch.cuda.synchronize()
+        assert torch.equal(runs[0], y)
     x = xs[:, :K].double()
     if norm:
         x = x * torch.rsqrt((x * x).mean(-1, keepdim=True) + 1e-6) * gain.double()

@@ -306,14 +306,24 @@ def test_ring_tile_refuses_ungated_linears(gpu):
     assert "ring" in mt.last_error()
 
 
+# More of them for fp32 x: whole 64-k stages run on the direct kernel (RING_SHAPES with K = 896 and
+# 320), so the ring kernel's own loop over many stages needs a K that is none.
+RING_SPLIT_SHAPES = [
+    (448, 4864, 904, O.SILU_GATE, False),             # the automatic choice; 15 stages, the last of 8 k
+    (150, 200, 2056, O.SILU_GATE | O.ACCUM, True),    # 33 stages; ragged rows and features
+    (129, 100, 1992, O.SILU_GATE, True),              # 32 stages
+]
+
+
 @pytest.mark.parametrize("norm", [False, True], ids=["plain", "rmsnorm"])
 @pytest.mark.parametrize("wt", [O.F16, O.BF16], ids=["wf16", "wbf16"])
-@pytest.mark.parametrize("shape", RING_SHAPES, ids=_ids)
+@pytest.mark.parametrize("shape", RING_SHAPES + RING_SPLIT_SHAPES, ids=_ids)
 def test_gated_ring_kernel_fp32_activations(gpu, shape, wt, norm):
-    """The gated ring kernel for fp32 x (hi + lo halves, MT_TUNE_GEMM_TILE = 5; the auto choice
-    for gated linears whose ring tiles fill at least 3/4 of their last wave), with and without
-    the fused RMSNorm, against the oracle's fp32 loop and fp64 within the split bound; re-run
-    bit-identical, and where the default routing takes it (gate|up at 512 rows) the same bits."""
+    """The gated tiles of 128 x 96 features for fp32 x (hi + lo halves, MT_TUNE_GEMM_TILE = 5; the auto
+    choice for gated linears whose tiles fill at least 3/4 of their last wave), on the direct kernel
+    for K of whole 64-k stages and the ring kernel otherwise, with and without the fused RMSNorm,
+    against the oracle's fp32 loop and fp64 within the split bound; re-run bit-identical, and where the
+    default routing takes these tiles (gate|up at 448 and 512 rows) the same bits."""
     M, N, K, flags, bias = shape
     say(f"ring fp32 x w{wt} norm={norm} {_ids(shape)}")
     c = _case(M * 23 + N + K + wt, M, N, K, flags, bias, wt)
