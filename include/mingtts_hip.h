@@ -182,11 +182,14 @@ enum {
                                     linears only: the auto choice when its tiles fill at least
                                     3/4 of their last wave on the CUs, e.g. gate|up at 448-640
                                     rows on 256 CUs; fp32 x of whole 64-k stages takes
-                                    these tiles on the direct kernel) */
+                                    these tiles on the direct kernel, by request at any such K up
+                                    to 2048 with a fused norm, by the auto choice at 512 <= K <
+                                    2048) */
     MT_TUNE_GEMM_STAGES = 7,     /* loads of that GEMM for x of the weights' type: 2..4 = direct-to-LDS
                                     stages of 64 k, 1 = two register-staged stages into two LDS
-                                    buffers (0 = auto); fp32 x always stages through registers,
-                                    its K loop 1 = committing only the split's stages, 2..4 = the
+                                    buffers (0 = auto); fp32 x stages through registers (the
+                                    direct kernel, which reads x straight into operands, is the auto
+                                    choice's only), its K loop 1 = committing only the split's stages, 2..4 = the
                                     branch-free loop (64-row tiles; 0 = auto) */
     MT_TUNE_GEMV_MFMA = 8,       /* the MFMA kernel that stages x once per 16 output features: 0 =
                                     for 3..16 rows (default; 3..8 with a fused norm), 1 = never

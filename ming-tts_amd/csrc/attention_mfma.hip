@@ -21,18 +21,18 @@
 //     three bf16 pieces (all 24 bits) and the 6 products above 2^-24.  Sums are fp32, but an MFMA
 //     rounds its sums towards zero, so the weights' sum takes the same way as p . v (ones in place of the
 //     values): the same rounded weights and nearly the same loss stand above and below the fraction.
-//     Normwise error against fp64 over that of the row kernel, fp16 / fp32 cache: 0.64-1.02 / 0.59-0.88
+//     Normwise error against fp64 over that of the row kernel, fp16 / fp32 cache: 0.64-1.04 / 0.59-0.88
 //     at 400 to 2048 rows, windows of 5 and 65 and none, queries of 0.1 to 40; values with a mean
 //     0.89-1.01 / 0.82-0.87 (1.3 / 1.05 with the weights summed beside the MFMAs, which takes 0.1-1 us
 //     less, 4 less at 4000 fp16 keys, and 1.1 more at 1600 fp16 rows of window 65).
 //   - Tiles start at multiples of 32 keys, a tile without keys of a row adds exact zeros to it, and
 //     the four waves' parts meet in wave order: a row's result does not depend on the block it falls
 //     into while the cache rows that the block reads are finite.
-//   - Bound: a wave's own instructions (about 240 a tile beside 16 MFMAs with an fp16 cache) and,
+//   - Bound: a wave's own instructions (about 240 vector instructions a tile with an fp16 cache, its 20
+//     MFMAs and a share of the set-up among them: MFMAs busy 25 % of the time, waves waiting 34 %) and,
 //     with few tiles a wave, its loads' latency.  2048 rows from position 0 (14 / 2 heads, graph
-//     replay): 31 us with an fp16 cache, 64 us with an fp32 one (row kernels 431 and 766).  Two row
-//     tiles a wave, which halve the key and value reads, took 256 registers and 36-59 us; three
-//     waves a SIMD spill (38 us).
+//     replay): 31 us with an fp16 cache, 66 us with an fp32 one (row kernels 432 and 771).  Two row
+//     tiles a wave, which halve the key and value reads, took 256 registers and 36-59 us.
 //   - A row with an output that is not finite (infinities and NaN in its query or keys, or in cache
 //     rows that it does not attend but its block reads) is done again with the row kernel's arithmetic,
 //     which touches only the row's own keys.

@@ -25,10 +25,11 @@
 //     with x through LDS as fp32 (direct loads) were bound by LDS writes instead and no faster
 //     (gate|up at 2048 rows 101 us), nor were persistent workgroups that load the next tile during the
 //     epilogue (97 us against 96-104).  Graph replay over six sets of operands, fp16 weights, against
-//     ring_split_kernel or tiled_kernel: rmsnorm+gate|up 117 -> 109 us at 2048 rows, 90 -> 80 at 1600,
-//     30.8 -> 25.8 at 512, 24.2 -> 17.6 at 256; rmsnorm+qkv 25.2 -> 18.3 at 2048; the DiT block's qkv
-//     25.8 -> 19.8 and ff1 27.7 -> 24.6 at 800.  One layer over 2048 rows 252 -> 243 us, the DiT block
-//     over 800 rows 107 -> 102 us.
+//     ring_split_kernel or tiled_kernel: rmsnorm+gate|up 115 -> 106 us at 2048 rows, 89 -> 79 at 1600,
+//     61 -> 52 at 1024, 30.9 -> 26.6 at 512, 25.4 -> 19.0 at 256; rmsnorm+qkv 26.4 -> 19.7 at 2048; the DiT
+//     block's qkv (bf16) 27.4 -> 22.0 and ff1 28.4 -> 27.3 at 800.  One layer over 2048 rows 252 -> 243
+//     us, the DiT block over 800 rows 107 -> 102 us.  MFMAs busy 29 % of the time (gate|up at 2048 rows),
+//     waves waiting 31 %, 71 % of the reads hit L2.
 #pragma once
 
 #include "tiled_kernel.hpp"

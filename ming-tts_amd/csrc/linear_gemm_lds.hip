@@ -123,8 +123,8 @@ size_t tiled_partial_bytes(const TiledPlan &p, bool gated, bool norm) {
 //   M = 704-768 (306 tiles, 0.60 of two)  32.3 / 54.6 against 21.9 / 45.3 (tiled)
 //   M = 1024 (408 tiles, 0.80 of two)     33.8 / 56.8 against 36.8 / 59.1
 // Below 384 rows (102 tiles or fewer) the tiled plans are faster as well.  fp32 x of whole 64-k stages
-// takes the same tiles on the direct kernel (linear_gemm_direct.hip): 24.5 us at 512 rows, 47.9 at 1024;
-// ring_split_kernel keeps other K.
+// takes the same tiles on the direct kernel (linear_gemm_direct.hip): 26.6 us at 512 rows, 52 at 1024;
+// ring_split_kernel keeps other K (fewer than 512, 2048 and more, or no whole stages).
 static bool ring_fills(uint32_t M, uint32_t N, int cus) {
     const uint64_t t = static_cast<uint64_t>((M + ring::BM - 1) / ring::BM) * ((N + ring::FN - 1) / ring::FN);
     const uint64_t c = static_cast<uint64_t>(cus > 0 ? cus : 256);
